@@ -15,7 +15,8 @@
 //   f32_to_bf16           activations for the bf16 grouped kernels behind the
 //                         reference-signature moe_expert_ffn_w4a16.
 //
-// The GEMVs are decode-shaped (the shared expert at small n): a workgroup of 4
+// Shapes of whole K chunks and output rows by 32 take the matrix cores
+// (splitmm.hpp); the GEMVs here take the others. They are decode-shaped (the shared expert at small n): a workgroup of 4
 // waves owns 16 output rows (4 per wave) and walks the tokens in blocks of 8.
 // Each 512-wide K chunk of the 8 token rows is staged once in LDS and shared
 // by the 4 waves; each lane then holds 8 consecutive K of its 4 rows (one
@@ -24,6 +25,7 @@
 // results are deterministic. Weights are read once per token block.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "splitmm.hpp"
 
 namespace glmmoe {
 
@@ -187,11 +189,27 @@ static int launch_ref_gemv(const float* x, const uint8_t* w, const float* sc, co
 
 int launch_ref_gemm_w4(const float* x, const uint8_t* qw, const float* sc, const float* bias,
                        float* y, int n, int in, int out, int g, hipStream_t s) {
+    // us at n = 1 / 8 / 64 / 203, 6144 -> 2048: 13 / 18 / 26 / 52 against 26 / 31 / 232 / 952 of ref_gemv_kernel
+    if (in % sm_kc(kSmW4) == 0 && g % 32 == 0 && in % g == 0 && out % 32 == 0 &&
+        ((uintptr_t)qw & 3) == 0 && ((uintptr_t)x & 15) == 0) {
+        SmArgs a{};
+        a.x = x; a.w0 = qw; a.rb0 = in / 2; a.sc = sc; a.group = g; a.bias = bias; a.y = y;
+        a.K = in; a.out = out; a.n = n;
+        return sm_dense<kSmW4>(false, a, s);
+    }
     return launch_ref_gemv<false>(x, qw, sc, bias, y, n, in, out, g, s);
 }
 
 int launch_ref_gemm_fp8(const float* x, const uint8_t* w, const float* sc, const float* bias,
                         float* y, int n, int in, int out, hipStream_t s) {
+    // us at n = 1 / 8 / 64 / 203, 6144 -> 2048: 11 / 16 / 26 / 53 against 48 / 54 / 407 / 1498 of ref_gemv_kernel
+    if (in % sm_kc(kSmFp8) == 0 && out % 32 == 0 && ((uintptr_t)w & 3) == 0 &&
+        ((uintptr_t)x & 15) == 0) {
+        SmArgs a{};
+        a.x = x; a.w0 = w; a.rb0 = in; a.sc = sc; a.group = in; a.bias = bias; a.y = y;
+        a.K = in; a.out = out; a.n = n;
+        return sm_dense<kSmFp8>(false, a, s);
+    }
     return launch_ref_gemv<true>(x, w, sc, bias, y, n, in, out, 1, s);
 }
 

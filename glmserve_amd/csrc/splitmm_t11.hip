@@ -1,0 +1,6 @@
+#include "splitmm_launch.hpp"
+
+namespace glmmoe {
+template int sm_moe<11>(bool, bool, int, const SmArgs&, unsigned, hipStream_t);
+template int sm_dense<11>(bool, const SmArgs&, hipStream_t);
+}  // namespace glmmoe

@@ -1,0 +1,126 @@
+"""The matrix-core products of fp32 / int8 rows with block-quantized weights
+(csrc/splitmm.hpp) behind gemm_q, gemm_q_i8, gemm_w4a16 and gemm_fp8, at the edges of their tiles, chunks
+and launch rules, against 64-bit products of the oracle's dequantized weights.
+
+Tolerance. Every output is a sum of K / 32 pieces (each a product of 32 terms
+added in fp32 by the matrix core), added in two levels of at most 16 and 24
+terms: in the 2-norm about sqrt(16 / 2 + 24 / 2 + 4) * 2^-24 / sqrt(3) = 1.7e-7
+of the result at most; 2.5e-7 is the bound (fp32 vector sums: the same order).
+Values with an offset per block (Q4_K, Q5_K: ds * q - dm) subtract two sums
+several times the result: four times that.
+"""
+import numpy as np
+import pytest
+import torch
+
+from glmserve_amd import ops
+from moe_cases import GGUF_TYPES, random_gguf_rows
+
+pytestmark = pytest.mark.gpu
+TYPES = [8, 11, 12, 13, 14, 18, 23]
+TOL = {t: 1e-6 if t in (12, 13) else 2.5e-7 for t in TYPES}
+
+
+def _dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _rows(t, rows, k, rng):
+    """GGUF rows with row_bytes rounded up to a multiple of 4 (dword-aligned rows)."""
+    w = random_gguf_rows(t, rows, k, rng)
+    pad = -w.shape[1] % 4
+    return np.concatenate([w, np.zeros((rows, pad), np.uint8)], 1), w
+
+
+def _err(got, ref):
+    assert np.isfinite(got).all()
+    return float(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+
+
+def _quant(x):
+    xq = torch.empty(x.shape, dtype=torch.int8, device="cuda")
+    xs = torch.empty(x.shape[0], x.shape[1] // 32, device="cuda")
+    ops.ref_quantize_act_q8(_dev(x), xq, xs)
+    q, s = xq.cpu().numpy(), xs.cpu().numpy()
+    return xq, xs, (q.reshape(len(x), -1, 32) * s.astype(np.float64)[:, :, None]).reshape(x.shape)
+
+
+# Tokens: the tiles of 4, 16 and 32 and their remainders; K: one chunk, an odd
+# number of chunks (the last one in the middle of a dword for the 2-byte aligned
+# types) and more chunks than the 8 K shares; outputs: one block, a remainder.
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("n,in_,out", [(1, 256, 32), (4, 1280, 96), (5, 768, 64), (16, 2304, 32),
+                                       (17, 1280, 160), (33, 256, 64)])
+def test_gemm(oracle, qtype, n, in_, out):
+    rng = np.random.default_rng(qtype * 100 + n)
+    wp, w = _rows(qtype, out, in_, rng)
+    W = oracle.gguf_dequant_rows(qtype, w, out, in_).astype(np.float64)
+    x = rng.standard_normal((n, in_)).astype(np.float32)
+    b = rng.standard_normal(out).astype(np.float32)
+    y = torch.full((n, out), float("nan"), device="cuda")
+    ops.ref_gemm_q(qtype, _dev(x), _dev(wp), _dev(b), y, wp.shape[1])
+    assert _err(y.cpu().numpy(), x.astype(np.float64) @ W.T + b) < TOL[qtype]
+    xq, xs, xd = _quant(x)
+    ops.ref_gemm_q_i8(qtype, xq, xs, _dev(wp), None, y, wp.shape[1])
+    assert _err(y.cpu().numpy(), xd @ W.T) < TOL[qtype]
+
+
+# 64-token x 256-row tiles: 7 x 28 workgroups, the last tile one token.
+@pytest.mark.parametrize("qtype", [8, 12, 18, 23])
+def test_gemm_large_tiles(oracle, qtype):
+    rng = np.random.default_rng(qtype)
+    n, in_, out = 385, 256, 7168 - 32
+    w = random_gguf_rows(qtype, out, in_, rng)
+    W = oracle.gguf_dequant_rows(qtype, w, out, in_).astype(np.float64)
+    x = rng.standard_normal((n, in_)).astype(np.float32)
+    y = torch.full((n, out), float("nan"), device="cuda")
+    wp = np.concatenate([w, np.zeros((out, -w.shape[1] % 4), np.uint8)], 1)
+    ops.ref_gemm_q(qtype, _dev(x), _dev(wp), None, y, wp.shape[1])
+    assert _err(y.cpu().numpy(), x.astype(np.float64) @ W.T) < TOL[qtype]
+    xq, xs, xd = _quant(x)
+    ops.ref_gemm_q_i8(qtype, xq, xs, _dev(wp), None, y, wp.shape[1])
+    assert _err(y.cpu().numpy(), xd @ W.T) < TOL[qtype]
+
+
+@pytest.mark.parametrize("n,in_,out,g", [(1, 256, 32, 32), (7, 768, 96, 96), (19, 512, 64, 512)])
+def test_gemm_w4_fp8(oracle, n, in_, out, g):
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n, in_)).astype(np.float32)
+    y = torch.full((n, out), float("nan"), device="cuda")
+    q = rng.integers(0, 256, (out, in_ // 2), dtype=np.uint8)
+    s = rng.uniform(0.001, 0.02, (out, in_ // g)).astype(np.float32)
+    W = oracle.dequant_int4_rows(q, s, in_, g).astype(np.float64)
+    ops.ref_gemm_w4a16(_dev(x), _dev(q), _dev(s), None, y, g)
+    assert _err(y.cpu().numpy(), x.astype(np.float64) @ W.T) < 2.5e-7
+    c = rng.integers(0, 256, (out, in_), dtype=np.uint8)
+    c[(c & 0x7F) == 0x7F] = 0x3C
+    sc = rng.uniform(0.5, 1.5, out).astype(np.float32)
+    W = np.array([oracle.e4m3_to_f32(v) for v in range(256)], np.float64)[c] * sc[:, None].astype(np.float64)
+    ops.ref_gemm_fp8(_dev(x), _dev(c), _dev(sc), None, y)
+    assert _err(y.cpu().numpy(), x.astype(np.float64) @ W.T) < 2.5e-7
+
+
+@pytest.mark.parametrize("qtype", [8, 18])
+def test_extreme_activations(oracle, qtype):
+    # Tokens of very large and very small rows keep their relative accuracy; an
+    # infinity or NaN stays in its token and gives what the fp32 product gives.
+    rng = np.random.default_rng(3 + qtype)
+    n, in_, out = 6, 512, 64
+    w = random_gguf_rows(qtype, out, in_, rng)
+    W = oracle.gguf_dequant_rows(qtype, w, out, in_).astype(np.float64)
+    x = rng.standard_normal((n, in_)).astype(np.float32)
+    x[1] *= np.float32(1e30)
+    x[2] *= np.float32(1e-25)
+    x[3, ::2] *= np.float32(1e-6)   # small terms beside large ones
+    x[4, 77] = -np.inf
+    x[5, 300] = np.nan
+    y = torch.zeros(n, out, device="cuda")
+    ops.ref_gemm_q(qtype, _dev(x), _dev(w), None, y, w.shape[1])
+    got = y.cpu().numpy()
+    ref = x[:4].astype(np.float64) @ W.T
+    for t in range(4):
+        assert _err(got[t], ref[t]) < 5e-7, t   # a norm over 64 outputs only
+    with np.errstate(invalid="ignore"):
+        inf = np.float32(-np.inf) * W[:, 77].astype(np.float32)   # NaN for a zero weight
+    assert np.array_equal(got[4], inf, equal_nan=True)
+    assert np.isnan(got[5]).all()
