@@ -1,5 +1,6 @@
 """The matrix-core products of fp32 / int8 rows with block-quantized weights
-(csrc/splitmm.hpp) behind gemm_q, gemm_q_i8, gemm_w4a16 and gemm_fp8, at the edges of their tiles, chunks
+(csrc/splitmm.hpp) behind gemm_q, gemm_q_i8, gemm_w4a16, gemm_fp8,
+moe_expert_ffn_q and moe_expert_ffn_q_i8, at the edges of their tiles, chunks
 and launch rules, against 64-bit products of the oracle's dequantized weights.
 
 Tolerance. Every output is a sum of K / 32 pieces (each a product of 32 terms
@@ -98,6 +99,61 @@ def test_gemm_w4_fp8(oracle, n, in_, out, g):
     W = np.array([oracle.e4m3_to_f32(v) for v in range(256)], np.float64)[c] * sc[:, None].astype(np.float64)
     ops.ref_gemm_fp8(_dev(x), _dev(c), _dev(sc), None, y)
     assert _err(y.cpu().numpy(), x.astype(np.float64) @ W.T) < 2.5e-7
+
+
+# E = 8, top-4: ungrouped (tiles of 4 with one row), then 12, 36 and 2080 routed
+# rows grouped (tiles of 8, 16 and 64; int8 and fp32), ids outside [0, E) among them.
+@pytest.mark.parametrize("types", [(18, 18, 23), (8, 8, 8), (12, 12, 13), (11, 11, 14), (23, 23, 18)])
+@pytest.mark.parametrize("n,grouped", [(3, False), (3, True), (9, True), (70, True), (520, True)])
+def test_moe(oracle, types, n, grouped):
+    H, I, E, k = 1024, 512, 8, 4
+    rng = np.random.default_rng(sum(types) + n)
+    geo = [(types[0], I, H), (types[1], I, H), (types[2], H, I)]
+    pk = [_rows(t, E * r, c, rng) for t, r, c in geo]
+    W = [oracle.gguf_dequant_rows(t, p[1], E * r, c).reshape(E, r, c).astype(np.float64)
+         for (t, r, c), p in zip(geo, pk)]
+    dev = [_dev(p[0]) for p in pk]
+    rb = tuple(p[0].shape[1] for p in pk)
+    # block scales are about 1e-2: keep gate and up of order one
+    x = (rng.standard_normal((n, H)) * 2e-2).astype(np.float32)
+    ids = np.stack([rng.permutation(E)[:k] for _ in range(n)]).astype(np.int32)
+    ids[rng.random((n, k)) < 0.1] = E
+    ids[0] = [0, 1, 2, -1]
+    w = rng.uniform(0.1, 1.0, (n, k)).astype(np.float32)
+    flat, tok = ids.reshape(-1), np.arange(n * k) // k
+
+    def ref_h(xd):
+        h = np.zeros((n * k, I))
+        for e in range(E):
+            r = np.nonzero(flat == e)[0]
+            g, u = xd[tok[r]] @ W[0][e].T, xd[tok[r]] @ W[1][e].T
+            h[r] = g / (1 + np.exp(-g)) * u
+        return h
+
+    def ref_out(h):
+        o = np.zeros((n, H))
+        for e in range(E):
+            r = np.nonzero(flat == e)[0]
+            np.add.at(o, tok[r], w.reshape(-1)[r][:, None] * (h[r] @ W[2][e].T))
+        return o
+
+    live = (flat >= 0) & (flat < E)
+    f = lambda *s: torch.zeros(*s, device="cuda")
+    h_act, dpart, out = f(n * k, I), f(n * k, H), f(n, H)
+    disp = torch.full((3 * E + 1 + n * k,), -7, dtype=torch.int32, device="cuda") if grouped else None
+    tol = 4 * max(TOL[t] for t in types)   # products of products
+    ops.ref_moe_expert_ffn_q(types, _dev(x), _dev(ids), _dev(w), *dev, I, E, rb, h_act, dpart, out, disp)
+    h = ref_h(x.astype(np.float64))
+    assert _err(h_act.cpu().numpy()[live], h[live]) < tol
+    assert _err(out.cpu().numpy(), ref_out(h)) < tol
+    # int8: gate/up from the quantized x, down from the quantized h it returns
+    xq, xs, xd = _quant(x)
+    hq, hs = torch.zeros(n * k, I, dtype=torch.int8, device="cuda"), f(n * k, I // 32)
+    ops.ref_moe_expert_ffn_q_i8(types, xq, xs, _dev(ids), _dev(w), *dev, I, E, rb, h_act, hq, hs, dpart,
+                                out, disp)
+    assert _err(h_act.cpu().numpy()[live], ref_h(xd)[live]) < tol
+    hd = hq.cpu().numpy().reshape(n * k, -1, 32) * hs.cpu().numpy().astype(np.float64)[:, :, None]
+    assert _err(out.cpu().numpy(), ref_out(hd.reshape(n * k, I))) < tol
 
 
 @pytest.mark.parametrize("qtype", [8, 18])
