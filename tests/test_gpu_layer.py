@@ -252,6 +252,16 @@ def test_large_group_other_shape(oracle, n):
     _check_full(out, oracle_full_w4(L, oracle, x, ids, w))
 
 
+@pytest.mark.parametrize("n", [332, 333])
+def test_group_size_threshold(oracle, n):
+    # 1660 and 1665 grouped rows: the last batch of the 16-row kernels (experts
+    # of several tiles, routing of a large batch) and the first of the 128-row ones.
+    L = SynthLayer(1024, 8, 4, 1024, seed=10)
+    x, out, logits, ids, w, offs, st, sr = _run(L, n, seed=n)
+    ref_logits = _check_routing(oracle, L, x, logits, ids, w, offs, st, sr)
+    _check_full(out, oracle_full_w4(L, oracle, x, ids, w))
+
+
 def test_split_last_round_deterministic():
     # Large-group batches whose gate/up last round runs as two K halves per
     # item (partials and a ticket per item; whichever half arrives second adds
