@@ -1288,11 +1288,135 @@ __global__ __launch_bounds__(kF32Threads) void router_logits_f32_kernel(
     }
 }
 
+// Larger batches: tiles of TT tokens x 32 experts, NW waves. The chains of the
+// chunks are independent until the fold, so each wave takes a chunk of its own
+// (chunk r * NW + w in round r): it stages 32 K of the tile's rows and weights
+// at a time into its own LDS ([k][row], rounded to bf16 and widened again, the
+// next 32 K loading meanwhile) and lane (tg, eq) runs TT / 8 tokens x 4 experts.
+// After a round the waves' partials go to LDS and every thread adds its
+// outputs' partials in chunk order. VALU-bound (one fma per product; two or
+// three LDS reads per 4 TT / 8 of them); a thread per (expert, chunk) and 8 tokens, as
+// above, converts every activation it uses and re-reads the weights per 8 tokens.
+constexpr int kF32TileE = 32, kF32TileK = 32, kF32Pad = 36;
+
+template <int TT, int NW>
+__global__ __launch_bounds__(64 * NW) void router_f32_tiled_kernel(
+    const float* __restrict__ x, const float* __restrict__ W, const float* __restrict__ bias,
+    float* __restrict__ y, int n, int H, int E) {
+    constexpr int MT = TT / 8, XL = TT / 8, WL = kF32TileE / 8;   // float4 loads per lane
+    constexpr int NOUT = TT * kF32TileE, NO = (NOUT + 64 * NW - 1) / (64 * NW);   // outputs per thread
+    __shared__ __align__(16) float xl[NW][kF32TileK][TT == 16 ? 20 : kF32Pad];
+    __shared__ __align__(16) float wl[NW][kF32TileK][kF32Pad];
+    __shared__ __align__(16) float part[NW][TT * kF32TileE];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int t0 = (int)blockIdx.y * TT, e0 = (int)blockIdx.x * kF32TileE;
+    const int nchunks = H / kRouterKC;
+    // Staging: lane = (row lane / 8 of 8, K quad lane % 8).
+    const int sr = lane >> 3, sk = lane & 7;
+    const float4 *xs[XL], *ws[WL];
+#pragma unroll
+    for (int j = 0; j < XL; ++j)
+        xs[j] = reinterpret_cast<const float4*>(x + (size_t)min(t0 + 8 * j + sr, n - 1) * H) + sk;
+#pragma unroll
+    for (int j = 0; j < WL; ++j)
+        ws[j] = reinterpret_cast<const float4*>(W + (size_t)min(e0 + 8 * j + sr, E - 1) * H) + sk;
+    float4 xv[XL], wv[WL];
+    auto load = [&](int k4) {   // K / 4
+#pragma unroll
+        for (int j = 0; j < XL; ++j) xv[j] = xs[j][k4];
+#pragma unroll
+        for (int j = 0; j < WL; ++j) wv[j] = ws[j][k4];
+    };
+    auto put = [&](float* base, int stride, int row, const float4& v) {
+        const uint32_t a = pack_bf16x2(v.x, v.y), b = pack_bf16x2(v.z, v.w);
+        float* p = base + 4 * sk * stride + row;
+        p[0] = __uint_as_float(a << 16);
+        p[stride] = __uint_as_float(a & 0xffff0000u);
+        p[2 * stride] = __uint_as_float(b << 16);
+        p[3 * stride] = __uint_as_float(b & 0xffff0000u);
+    };
+    constexpr int XS = sizeof(xl[0][0]) / 4;
+    const int tg = lane >> 3, eq = lane & 7;
+    float tot[NO];
+#pragma unroll
+    for (int i = 0; i < NO; ++i) tot[i] = 0.0f;
+    const int rounds = (nchunks + NW - 1) / NW;
+    load(min(wave, nchunks - 1) * (kRouterKC / 4));
+    for (int r = 0; r < rounds; ++r) {
+        const int c = min(r * NW + wave, nchunks - 1), cn = min((r + 1) * NW + wave, nchunks - 1);
+        float acc[MT][4];
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
+        for (int st = 0; st < kRouterKC / kF32TileK; ++st) {
+            // the wave's own buffers: its earlier reads precede these writes in order
+#pragma unroll
+            for (int j = 0; j < XL; ++j) put(&xl[wave][0][0], XS, 8 * j + sr, xv[j]);
+#pragma unroll
+            for (int j = 0; j < WL; ++j) put(&wl[wave][0][0], kF32Pad, 8 * j + sr, wv[j]);
+            load(st + 1 < kRouterKC / kF32TileK ? (c * kRouterKC + (st + 1) * kF32TileK) / 4
+                                                : cn * (kRouterKC / 4));
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll 8
+            for (int k = 0; k < kF32TileK; ++k) {
+                float xf[MT];
+#pragma unroll
+                for (int i = 0; i < MT; ++i) xf[i] = xl[wave][k][tg * MT + i];
+                const float4 w4 = *reinterpret_cast<const float4*>(&wl[wave][k][eq * 4]);
+                const float wf[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(xf[i], wf[j], acc[i][j]);
+            }
+            asm volatile("" ::: "memory");
+        }
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            *reinterpret_cast<float4*>(&part[wave][(tg * MT + i) * kF32TileE + eq * 4]) =
+                make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
+        __syncthreads();
+        const int live = min(NW, nchunks - r * NW);
+#pragma unroll
+        for (int i = 0; i < NO; ++i)
+            for (int w = 0; w < live; ++w)
+                tot[i] = tot[i] + part[w][min(tid + i * 64 * NW, NOUT - 1)];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < NO; ++i) {
+        const int o = tid + i * 64 * NW, t = t0 + o / kF32TileE, e = e0 + o % kF32TileE;
+        if (o < NOUT && t < n && e < E) y[(size_t)t * E + e] = bias ? tot[i] + bias[e] : tot[i];
+    }
+}
+
 int launch_router_logits_f32(const float* x, const float* W, const float* bias, float* y, int n,
                              int H, int E, hipStream_t s) {
     if (H % kRouterKC || H / kRouterKC > kF32Threads || H > 8192) return -2;
     const int nchunks = H / kRouterKC;
     const int epw = kF32Threads / nchunks;
+    const long blocks = (long)((E + epw - 1) / epw) * ((n + kRouterTG - 1) / kRouterTG);
+    // The thread-per-chunk kernel holds up to one workgroup per CU (H 6144, E
+    // 256: 64 tokens 28 us against 41 tiled, 96 tokens 52 against 41, 203: 80 /
+    // 42, 1000: 328 / 70, 4096: 1299 / 263) and, where a row has few chunks, up
+    // to one token group (H 2048, E 32, 8 to 1000 tokens: 20 against 15; H 256,
+    // E 16: 17 against 9). Tiles of 32 tokens once those of 16 exceed one per CU
+    // (512 tokens: 66 against 44 for 16, 1000: 70 against 85).
+    if (blocks > 256 || (nchunks <= 16 && n >= kRouterTG)) {
+        const unsigned eb = (unsigned)((E + kF32TileE - 1) / kF32TileE), t16 = (unsigned)((n + 15) / 16);
+        if ((long)t16 * eb > 256)
+            hipLaunchKernelGGL((router_f32_tiled_kernel<32, 8>), dim3(eb, (unsigned)((n + 31) / 32)), dim3(512),
+                               0, s, x, W, bias, y, n, H, E);
+        else if (nchunks > 8)
+            hipLaunchKernelGGL((router_f32_tiled_kernel<16, 16>), dim3(eb, t16), dim3(1024), 0, s, x, W, bias, y,
+                               n, H, E);
+        else
+            hipLaunchKernelGGL((router_f32_tiled_kernel<16, 8>), dim3(eb, t16), dim3(512), 0, s, x, W, bias, y, n,
+                               H, E);
+        return hipGetLastError() == hipSuccess ? 0 : -4;
+    }
     static bool attr_set = false;
     if (!attr_set) {
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(&router_logits_f32_kernel),

@@ -139,6 +139,23 @@ def test_router_logits_f32_bit_exact(oracle):
         assert np.array_equal(yb.cpu().numpy().view(np.uint32), (ref + bias[None, :]).view(np.uint32)), (n, H, E)
 
 
+# The tiled kernel's launch shapes: one round of chunks with idle waves, several
+# rounds with a partial last one, ragged token and expert tiles.
+@pytest.mark.parametrize("n,H,E", [(9, 256, 16), (40, 1920, 33), (96, 6144, 256), (203, 8192, 100),
+                                   (1030, 384, 130), (1030, 2304, 130)])
+def test_router_logits_f32_tiled_bit_exact(oracle, n, H, E):
+    rng = np.random.default_rng(n + H)
+    x = rng.standard_normal((n, H)).astype(np.float32)
+    w = (0.02 * rng.standard_normal((E, H))).astype(np.float32)
+    x[0, :4] = [1.0 + 2.0 ** -8, -(1.0 + 3 * 2.0 ** -9), 1e-39, -0.0]   # ties to even, a subnormal
+    bias = rng.uniform(-0.1, 0.1, E).astype(np.float32)
+    y = torch.full((n, E), float("nan"), dtype=torch.float32, device="cuda")
+    G.router_logits_f32(torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda(),
+                        torch.from_numpy(bias).cuda(), y)
+    ref = oracle.router_logits_bf16(oracle.f32_to_bf16(x), oracle.f32_to_bf16(w)) + bias[None, :]
+    assert np.array_equal(y.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+
+
 @pytest.mark.parametrize("n", [256, 520, 1000, 4096])
 def test_layer_routing_bit_exact_large_batches(oracle, n):
     """From 256 tokens the layer routes with MFMA logits plus an exact
