@@ -426,20 +426,31 @@ __device__ __forceinline__ void gg_dots_stream(GgStream<T, NM, TT, I8>& L, int* 
     }
 }
 
-// quantize_act_q8 (cuda/qgemm.cu:556-587): per 32-element block (one half
-// wave), sx = absmax / 127, q = round-half-even(v * (1 / sx)), 0 when sx = 0.
+// quantize_act_q8 (cuda/qgemm.cu:556-587): per 32-element block,
+// sx = absmax / 127, q = round-half-even(v * (1 / sx)), 0 when sx = 0. V
+// consecutive elements per thread (4 where x is 16-byte and xq 4-byte aligned),
+// 32 / V lanes per block. HBM-bound: 16.8 M elements 56 -> 19 us for V 4 against 1.
+template <int V>
 __global__ __launch_bounds__(256) void gg_quant_q8_kernel(const float* __restrict__ x, long total,
                                                           int8_t* __restrict__ xq,
                                                           float* __restrict__ xs) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const float v = i < total ? x[i] : 0.0f;
-    float a = fabsf(v);
+    const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * V;
+    typedef float vec __attribute__((ext_vector_type(V)));
+    vec v = 0.0f;
+    if (i < total) v = *reinterpret_cast<const vec*>(x + i);   // total is a multiple of 32
+    float a = fabsf(v[0]);
 #pragma unroll
-    for (int m = 16; m >= 1; m >>= 1) a = fmaxf(a, __shfl_xor(a, m));
+    for (int j = 1; j < V; ++j) a = fmaxf(a, fabsf(v[j]));
+#pragma unroll
+    for (int m = 16 / V; m >= 1; m >>= 1) a = fmaxf(a, __shfl_xor(a, m));
     if (i >= total) return;
     const float sx = a / 127.0f;
     const float id = sx > 0.0f ? 1.0f / sx : 0.0f;
-    xq[i] = (int8_t)(int)rintf(v * id);
+    typedef int8_t qvec __attribute__((ext_vector_type(V)));
+    qvec q;
+#pragma unroll
+    for (int j = 0; j < V; ++j) q[j] = (int8_t)(int)rintf(v[j] * id);
+    *reinterpret_cast<qvec*>(xq + i) = q;
     if ((i & 31) == 0) xs[i / 32] = sx;
 }
 
@@ -632,20 +643,26 @@ __global__ __launch_bounds__(kGgThreads) void gg_moe_kernel(GgMoeArgs a) {
 
 // out[t] = ((0 + w0 y0) + w1 y1) + ... over the slots (cuda/qgemm.cu:943-955).
 // Slots whose id is outside [0, E) add nothing (their dpart rows are never
-// written).
+// written). V outputs per thread (4: H % 4 == 0 and 16-byte aligned rows), the
+// slots' ids and weights uniform per workgroup: HBM-bound; 1000 tokens x top-8
+// x 6144 (221 MB) 100 -> 41 us against one output per thread.
+template <int V>
 __global__ __launch_bounds__(256) void gg_reduce_kernel(const float* __restrict__ dpart,
                                                         const int* __restrict__ ids,
-                                                        const float* __restrict__ w, int n,
-                                                        int topk, int H, int E, float* __restrict__ out) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)n * H) return;
-    const long t = i / H, o = i % H;
-    float acc = 0.0f;
+                                                        const float* __restrict__ w, int topk, int H,
+                                                        int E, float* __restrict__ out) {
+    const size_t t = blockIdx.x;
+    const int o = (int)(blockIdx.y * 256 + threadIdx.x) * V;
+    if (o >= H) return;
+    typedef float vec __attribute__((ext_vector_type(V)));
+    vec acc = 0.0f;
     for (int s = 0; s < topk; ++s) {
         const int e = ids[t * topk + s];
-        if (e >= 0 && e < E) acc = acc + w[t * topk + s] * dpart[(t * topk + s) * H + o];
+        if (e < 0 || e >= E) continue;
+        const vec v = *reinterpret_cast<const vec*>(dpart + (t * topk + s) * H + o);
+        acc = acc + w[t * topk + s] * v;
     }
-    out[i] = acc;
+    *reinterpret_cast<vec*>(out + t * H + o) = acc;
 }
 
 // Groups the routed rows by expert (one workgroup): d = [offsets E+1 | tile
@@ -827,8 +844,12 @@ int launch_gg_gemm_i8(uint32_t qtype, const int8_t* xq, const float* xs, const u
 }
 
 int launch_gg_quant_q8(const float* x, long total, int8_t* xq, float* xs, hipStream_t s) {
-    hipLaunchKernelGGL(gg_quant_q8_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
-                       x, total, xq, xs);
+    if (((uintptr_t)x & 15) == 0 && ((uintptr_t)xq & 3) == 0)
+        hipLaunchKernelGGL(gg_quant_q8_kernel<4>, dim3((unsigned)((total + 1023) / 1024)), dim3(256), 0, s, x,
+                           total, xq, xs);
+    else
+        hipLaunchKernelGGL(gg_quant_q8_kernel<1>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, x,
+                           total, xq, xs);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
@@ -864,9 +885,13 @@ static int gg_moe_phases(uint32_t gt, uint32_t ut, uint32_t dt, const GgMoeArgs&
 }
 
 static int gg_reduce(const GgMoeArgs& a, float* out, hipStream_t s) {
-    const long total = (long)a.n * a.H;
-    hipLaunchKernelGGL(gg_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a.dpart,
-                       a.ids, a.w, a.n, a.topk, a.H, a.E, out);
+    const bool v4 = a.H % 4 == 0 && (((uintptr_t)a.dpart | (uintptr_t)out) & 15) == 0;
+    const int per = v4 ? 1024 : 256;
+    const dim3 grid((unsigned)a.n, (unsigned)((a.H + per - 1) / per));
+    if (v4)
+        hipLaunchKernelGGL(gg_reduce_kernel<4>, grid, dim3(256), 0, s, a.dpart, a.ids, a.w, a.topk, a.H, a.E, out);
+    else
+        hipLaunchKernelGGL(gg_reduce_kernel<1>, grid, dim3(256), 0, s, a.dpart, a.ids, a.w, a.topk, a.H, a.E, out);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 

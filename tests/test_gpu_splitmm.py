@@ -180,3 +180,29 @@ def test_extreme_activations(oracle, qtype):
         inf = np.float32(-np.inf) * W[:, 77].astype(np.float32)   # NaN for a zero weight
     assert np.array_equal(got[4], inf, equal_nan=True)
     assert np.isnan(got[5]).all()
+
+
+def test_unaligned_elementwise(oracle):
+    # quantize_act_q8 and the combine on rows that are not 16-byte aligned.
+    rng = np.random.default_rng(8)
+    n, k, I, H, E, topk = 5, 96, 256, 512, 8, 4
+    x = rng.standard_normal((n, k)).astype(np.float32)
+    xf = torch.zeros(n * k + 1, device="cuda")
+    xf[1:] = _dev(x.reshape(-1))
+    xq, xs = torch.zeros(n * k + 1, dtype=torch.int8, device="cuda"), torch.zeros(n, k // 32, device="cuda")
+    ops.ref_quantize_act_q8(xf[1:].view(n, k), xq[1:].view(n, k), xs)
+    q, s = oracle.quant_act_q8(x)
+    assert np.array_equal(xq[1:].cpu().numpy().reshape(n, k), q) and np.array_equal(xs.cpu().numpy(), s)
+    g = _dev(random_gguf_rows(8, E * I, H, rng))
+    d = _dev(random_gguf_rows(8, E * H, I, rng))
+    x = _dev(rng.standard_normal((n, H)).astype(np.float32) * 0.02)
+    ids = _dev(np.stack([rng.permutation(E)[:topk] for _ in range(n)]).astype(np.int32))
+    w = _dev(rng.uniform(0.1, 1.0, (n, topk)).astype(np.float32))
+    outs = []
+    for off in (0, 1):
+        dpart = torch.zeros(n * topk * H + off, device="cuda")[off:]
+        out = torch.zeros(n, H, device="cuda")
+        ops.ref_moe_expert_ffn_q((8, 8, 8), x, ids, w, g, g, d, I, E, (H // 32 * 34, H // 32 * 34, I // 32 * 34),
+                                 torch.zeros(n * topk, I, device="cuda"), dpart, out, None)
+        outs.append(out.cpu())
+    assert torch.equal(outs[0], outs[1]) and float(outs[0].abs().sum()) > 0
