@@ -290,7 +290,12 @@ __global__ __launch_bounds__(256) void ref_silu_mul_kernel(const float* __restri
                                                            const float* __restrict__ u,
                                                            float* __restrict__ o, long n) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) o[i] = silu_f32(g[i]) * u[i];
+    // In 64 bits (2 M elements 6.4 -> 7.3 us, under a microsecond at decode): the
+    // int8 chain quantizes the result, and a rounding error there moves codes.
+    if (i < n) {
+        const double v = g[i];
+        o[i] = (float)(v / (1.0 + exp(-v)) * u[i]);
+    }
 }
 
 __global__ __launch_bounds__(256) void ref_add_inplace_kernel(float* __restrict__ y,

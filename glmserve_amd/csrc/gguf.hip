@@ -900,14 +900,22 @@ static int gg_reduce(const GgMoeArgs& a, float* out, hipStream_t s) {
 // and up of different types), or too little work for its 64-row workgroups.
 // The choice among tiles depends on the rows per expert (nk / E), which the
 // host knows only on average. Measured on the 6144 x 2048 x 256 layer, top-8,
-// IQ3_XXS / IQ4_XS (us for tiles of 4 / 8 / 16 / 64 rows, and before):
-//   fp32  n = 16: 601 / 704 / 836 / - (791); 64: 1240 / 1168 / 1382 / 1962
-//         (2303); 256: 3784 / 2590 / 1984 / 2671 (8815); 1000: 13042 / 7873 /
-//         5319 / 3974 (27440)
-//   int8  n = 16: 504 / 518 / 593 / - (650); 64: 970 / 855 / 983 / 1257 (1681);
-//         256: - / 1861 / 1401 / 1708 (2705); 1000: - / 5432 / 3647 / 2528 (3837)
-// The 64-row tile pays later for the K-quants (more decode per tile) and not
-// at all for the types with a scale per 16 K (see sm_dense_i). int8 calls below
+// IQ3_XXS / IQ4_XS (us for tiles of 4 / 8 / 16 / 32 / 64 rows, and before):
+//   fp32  n = 16: 601 / 704 / 836 / - / - (791); 64: 1240 / 1168 / 1382 / - /
+//         1962 (2303); 128: - / 1705 / 1631 / 1636 / 2155 (4202); 256: - / 2590 /
+//         2249 / 1895 / 2713 (8815); 1000: - / 8001 / 5304 / 3575 / 3942 (27440)
+//   int8  n = 16: 504 / 518 / 593 / - / - (650); 64: 970 / 855 / 983 / - / 1257
+//         (1681); 256: - / 1861 / 1378 / 1437 / 1665 (2705); 512: - / 3134 / 2142 /
+//         1877 / 1889; 1000: - / 5310 / 3544 / 2636 / 2406 (3837)
+// With the rows on a few hot experts (Zipf 1.1) or narrow experts the larger
+// tile wins earlier (int8 n = 256: 907 / 705 / 671 for 16 / 32 / 64). The
+// 64-row tile has fewer, larger steps and 256 registers full: int8 takes it
+// from 16 rows per expert, fp32 only where every expert has several (64), Q8_0
+// with fp32 rows never (1000: 4122 against 6492). The K-quants decode more per
+// tile: 16 rows up to 16 per expert (Q4_K, Q4_K, Q6_K, n = 256: 3176 / 3581,
+// 1000: 8517 / 6539), and the types with a scale per 16 K take the one-wave
+// sums of the larger tiles only up to K 4096, where their rounding error is not
+// above the vector kernels'. int8 calls below
 // 2048 routed rows stay on the small tiles, whose sums do not depend on the
 // tile: grouped and ungrouped calls agree bit for bit there.
 // Too little work: the vector kernels' 16-row workgroups win at n = 1 of that
@@ -927,9 +935,14 @@ static int gg_sm_tile(const GgMoeArgs& a, bool grouped) {
     if (nk <= E && work < (iq ? 24576 : 2048)) return 0;
     if (!grouped || nk <= E) return 4;
     if (nk <= 4 * E) return 8;
-    const bool g16 = sm_g16(gt) || sm_g16(dt);
-    const int large = iq ? (I8 ? 8 : 16) : gt == 8 && I8 ? 8 : 32;
-    return g16 || nk <= large * E || (I8 && nk < 2048) ? 16 : kSmLargeTile;
+    if (I8 && nk < 2048) return 16;
+    auto kquant = [](uint32_t t) { return t >= 11 && t <= 14; };
+    if (kquant(gt) || kquant(dt)) {
+        const bool long16 = (sm_g16(gt) && a.H > 4096) || (sm_g16(dt) && a.I > 4096);
+        return nk <= 16 * E || long16 ? 16 : kSmMidTile;
+    }
+    if (I8) return nk <= 16 * E ? kSmMidTile : kSmLargeTile;
+    return nk <= 64 * E || gt == 8 || dt == 8 ? kSmMidTile : kSmLargeTile;
 }
 
 // Gate/up and down on splitmm_kernel; d: the grouping in tiles of `tile` rows.

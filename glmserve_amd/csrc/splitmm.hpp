@@ -47,6 +47,8 @@
 
 #include <stddef.h>
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "gguf_dec.hpp"
 
@@ -72,8 +74,8 @@ struct SmArgs {
     const int* d;                   // MoE: grouping [offsets | tile prefix | rows], or null: row g alone
 };
 
-// Tokens per tile of the large MoE launch; the small ones take 4, 8 or 16.
-constexpr int kSmLargeTile = 64;
+// Tokens per tile of the large MoE launches; the small ones take 4, 8 or 16.
+constexpr int kSmMidTile = 32, kSmLargeTile = 64;
 // The launches (splitmm_launch.hpp): tile = tokens per tile of the grouping.
 template <uint32_t T>
 int sm_moe(bool down, bool i8, int tile, const SmArgs& a, unsigned tiles, hipStream_t s);
@@ -550,7 +552,16 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
     // The A row of this lane holds tile token ta (+ 32 tb).
     const int ta = SM ? (lr >> 2) * NV + (lr & (NV - 1)) : lr;
     const int ntb = TB == 1 ? 1 : __builtin_amdgcn_readfirstlane((nr + 31) / 32);
-    float acc[NK][TB][NV], part[NK][TB][NV];
+    // int8 products mostly feed the int8 quantizer again, where one rounding more
+    // or less moves a code: up to 16 rows per expert (gate/up) and in the linears'
+    // tiles of at most 32 tokens the exact integer dots are scaled and added in
+    // 64 bits (a fused multiply-add costs the same), so the result is the rounded
+    // exact value: the int8 layer's error against 64 bits 5e-5 -> 1.3e-7, 64
+    // tokens 855 -> 873 us.
+    constexpr bool F64 = I8 && ((SM && MODE == kSmGateUp) || (TB == 1 && MODE == kSmDense));
+    using Acc = std::conditional_t<F64, double, float>;
+    Acc acc[NK][TB][NV];
+    float part[NK][TB][NV];
 #pragma unroll
     for (int nb = 0; nb < NK; ++nb)
 #pragma unroll
@@ -619,20 +630,24 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
             for (int h = 0; h < HV; ++h) ds[h] = scale_of(nb, HV * ib + h);
             if constexpr (I8) {
                 const sm_i32x2 w = sm_codes_i8<T>(rb_, ib, lq, skew, L.tab);
-                float v[NV];
+                Acc v[NV];
 #pragma unroll
                 for (int h = 0; h < HV; ++h) {
                     const bool mine = HV == 1 || (lq >> 1) == h;
                     const long B = __builtin_bit_cast(long, (sm_i32x2){mine ? w.x : 0, mine ? w.y : 0});
                     const sm_i32x4 D = __builtin_amdgcn_mfma_i32_16x16x32_i8(Ai, B, sm_i32x4{}, 0, 0, 0);
 #pragma unroll
-                    for (int i = 0; i < NV; ++i)
-                        v[i] = h ? __builtin_fmaf(ds[h], (float)D[i], v[i]) : ds[h] * (float)D[i];
+                    for (int i = 0; i < NV; ++i) {
+                        if constexpr (F64) v[i] = h ? __builtin_fma((double)ds[h], (double)D[i], v[i])
+                                                    : (double)ds[h] * (double)D[i];
+                        else v[i] = h ? __builtin_fmaf(ds[h], (float)D[i], v[i]) : ds[h] * (float)D[i];
+                    }
                 }
 #pragma unroll
                 for (int i = 0; i < NV; ++i) {
-                    if constexpr (sm_min(T)) v[i] = v[i] - L.dm[wave][nb * BR + lr][ib] * sxv[i];
-                    part[nb][0][i] = __builtin_fmaf(xsv[i], v[i], part[nb][0][i]);
+                    if constexpr (sm_min(T)) v[i] = v[i] - (Acc)L.dm[wave][nb * BR + lr][ib] * (Acc)sxv[i];
+                    if constexpr (F64) acc[nb][0][i] = __builtin_fma((double)xsv[i], v[i], acc[nb][0][i]);
+                    else part[nb][0][i] = __builtin_fmaf(xsv[i], v[i], part[nb][0][i]);
                 }
             } else {
                 const u32x4 w = sm_codes_bf16<T>(rb_, ib, lq, skew, L.tab);
@@ -683,7 +698,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
                 if constexpr (sm_min(T)) tokv(&L.xsum[kw][b][0], tb, sxv);
 #pragma unroll
                 for (int nb = 0; nb < NK; ++nb) {
-                    float v[NV];
+                    Acc v[NV];
 #pragma unroll
                     for (int h = 0; h < HV; ++h) {
                         sm_i32x16 D;
@@ -696,15 +711,19 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
                                 *reinterpret_cast<const sm_i32x4*>(ax + 16 * hh),
                                 (sm_i32x4){w[nb][0].x, w[nb][0].y, w[nb][1].x, w[nb][1].y}, sm_i32x16{}, 0, 0, 0);
 #pragma unroll
-                        for (int i = 0; i < NV; ++i)
-                            v[i] = h ? __builtin_fmaf(ds[nb][h], (float)D[i], v[i]) : ds[nb][h] * (float)D[i];
+                        for (int i = 0; i < NV; ++i) {
+                            if constexpr (F64) v[i] = h ? __builtin_fma((double)ds[nb][h], (double)D[i], v[i])
+                                                        : (double)ds[nb][h] * (double)D[i];
+                            else v[i] = h ? __builtin_fmaf(ds[nb][h], (float)D[i], v[i]) : ds[nb][h] * (float)D[i];
+                        }
                     }
                     float dmv = 0.0f;
                     if constexpr (sm_min(T)) dmv = L.dm[wave][nb * BR + lr][ib];
 #pragma unroll
                     for (int i = 0; i < NV; ++i) {
-                        if constexpr (sm_min(T)) v[i] = v[i] - dmv * sxv[i];
-                        part[nb][tb][i] = __builtin_fmaf(xsv[i], v[i], part[nb][tb][i]);
+                        if constexpr (sm_min(T)) v[i] = v[i] - (Acc)dmv * (Acc)sxv[i];
+                        if constexpr (F64) acc[nb][tb][i] = __builtin_fma((double)xsv[i], v[i], acc[nb][tb][i]);
+                        else part[nb][tb][i] = __builtin_fmaf(xsv[i], v[i], part[nb][tb][i]);
                     }
                 }
             }
@@ -756,8 +775,9 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
     };
 
     const int iters = (nch + KW - 1) / KW;
-    // Chunks per inner sum: 256 K, 512 where one wave walks all of K.
-    constexpr int FL = (KW == 1 ? 512 : 256) / KC;
+    // Chunks per inner sum: 256 K, 512 where one wave walks a long K (the two
+    // levels then have about as many terms).
+    const int FL = (KW == 1 && K > 4096 ? 512 : 256) / KC;
     load_x(min(kw, nch - 1) * KC);
     for (int it = 0; it < iters; ++it) {
         const int c = it * KW + kw;
@@ -768,7 +788,9 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
         const uint8_t* const brow = raw + lr * RS + skew;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if constexpr (T != kSmFp8) scales(raw + skew, cc);
-#pragma unroll
+        // 32-token tiles: one step of code, or the scheduler hoists several
+        // steps' decodes and spills
+#pragma unroll(NT == 32 && RW > 1 ? 1 : ST)
         for (int s = 0; s < ST; ++s) {
             if constexpr (RW == 1) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             else sm_barrier();
@@ -789,7 +811,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
                 }
             }
         }
-        if ((it + 1) % FL == 0 || it + 1 == iters) {
+        if (!F64 && ((it + 1) % FL == 0 || it + 1 == iters)) {
 #pragma unroll
             for (int nb = 0; nb < NK; ++nb)
 #pragma unroll
@@ -805,9 +827,9 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
     if constexpr (KW > 1) {
         // The shares' sums, added in pairs; the staging buffers are free by then.
         constexpr int AV = NK * TB * NV;
-        static_assert(sizeof(float) * (KW - 1) * RW * AV * 64 <= sizeof(S) - offsetof(S, x),
+        static_assert(sizeof(Acc) * (KW - 1) * RW * AV * 64 <= sizeof(S) - offsetof(S, x),
                       "share sums fit the staging buffers");
-        float* red = reinterpret_cast<float*>(&L.x[0][0][0][0]);
+        Acc* red = reinterpret_cast<Acc*>(&L.x[0][0][0][0]);
         sm_barrier();
         if (kw > 0) {
 #pragma unroll
@@ -819,8 +841,8 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
         if (kw > 0) return;
 #pragma unroll
         for (int v = 0; v < AV; ++v) {
-            float& o = acc[v / (TB * NV)][v / NV % TB][v % NV];
-            float p[KW];
+            Acc& o = acc[v / (TB * NV)][v / NV % TB][v % NV];
+            Acc p[KW];
             p[0] = o;
 #pragma unroll
             for (int q = 1; q < KW; ++q) p[q] = red[(((q - 1) * RW + rw) * AV + v) * 64 + lane];
@@ -843,8 +865,10 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
                 if (f0 + 32 > a.out) continue;
 #pragma unroll
                 for (int nb = 0; nb < NK / 2; ++nb) {
-                    const float g = acc[nb][tb][i], u = acc[nb + NK / 2][tb][i];
-                    a.y[(size_t)L.row[t] * a.out + f0 + nb * BR + lr] = g / (1.0f + expf(-g)) * u;
+                    const Acc g = acc[nb][tb][i], u = acc[nb + NK / 2][tb][i];
+                    float& h = a.y[(size_t)L.row[t] * a.out + f0 + nb * BR + lr];
+                    if constexpr (F64) h = (float)(g / (1.0 + exp(-g)) * u);
+                    else h = g / (1.0f + expf(-g)) * u;
                 }
             } else {
                 const size_t r = MODE == kSmDown ? (size_t)L.row[t] : (size_t)(t0 + t);
@@ -852,7 +876,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
                 for (int nb = 0; nb < NK; ++nb) {
                     const int o = f0 + nb * BR;
                     if (f0 + 32 * (nb * BR / 32) + 32 > a.out) continue;
-                    float v = acc[nb][tb][i];
+                    float v = (float)acc[nb][tb][i];
                     if constexpr (MODE == kSmDense) {
                         if constexpr (T == kSmFp8) v = a.sc ? v * a.sc[o + lr] : v;
                         if (a.bias) v += a.bias[o + lr];

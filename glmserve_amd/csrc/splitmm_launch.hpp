@@ -7,7 +7,7 @@
 namespace glmmoe {
 
 // MoE launches: the small tiles (4, 8, 16 tokens) split K over the workgroup's
-// four waves, the large one (64) its weight rows.
+// four waves, the others (32, 64) its weight rows.
 template <uint32_t T, int MODE, bool I8, int RW, int KW, int NB, int NT, int KX>
 static int sm_go(const SmArgs& a, unsigned gx, hipStream_t s) {
     constexpr int rows = (MODE == kSmGateUp ? 32 : 32 * NB) * RW;
@@ -27,6 +27,8 @@ template <uint32_t T, int MODE, bool I8>
 static int sm_moe_mode(int tile, const SmArgs& a, unsigned tiles, hipStream_t s) {
     if (tile == 4) return sm_go<T, MODE, I8, 1, 4, 2, 4, sm_kx(T, 4)>(a, tiles, s);
     if (tile == 8) return sm_go<T, MODE, I8, 1, 4, 2, 8, sm_kx(T, 8)>(a, tiles, s);
+    if (tile == kSmMidTile)
+        return sm_go<T, MODE, I8, 4, 1, 2, 32, I8 || T == 8 ? 128 : T == 14 ? 32 : 64>(a, tiles, s);
     if constexpr (!sm_g16(T)) {
         if (tile == kSmLargeTile) return sm_go<T, MODE, I8, 4, 1, 2, 64, I8 ? 128 : sm_kx(T, 64)>(a, tiles, s);
     }

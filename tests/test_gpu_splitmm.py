@@ -101,8 +101,8 @@ def test_gemm_w4_fp8(oracle, n, in_, out, g):
     assert _err(y.cpu().numpy(), x.astype(np.float64) @ W.T) < 2.5e-7
 
 
-# E = 8, top-4: ungrouped (tiles of 4 with one row), then 12, 36 and 2080 routed
-# rows grouped (tiles of 8, 16 and 64; int8 and fp32), ids outside [0, E) among them.
+# E = 8, top-4: ungrouped (tiles of 4 with one row), then 12, 36, 280 and 2080
+# routed rows grouped (tiles of 8, 16 or 32, 32 and 64), ids outside [0, E) among them.
 @pytest.mark.parametrize("types", [(18, 18, 23), (8, 8, 8), (12, 12, 13), (11, 11, 14), (23, 23, 18)])
 @pytest.mark.parametrize("n,grouped", [(3, False), (3, True), (9, True), (70, True), (520, True)])
 def test_moe(oracle, types, n, grouped):
