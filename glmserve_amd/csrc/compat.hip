@@ -190,7 +190,7 @@ static int launch_ref_gemv(const float* x, const uint8_t* w, const float* sc, co
 int launch_ref_gemm_w4(const float* x, const uint8_t* qw, const float* sc, const float* bias,
                        float* y, int n, int in, int out, int g, hipStream_t s) {
     // us at n = 1 / 8 / 64 / 203, 6144 -> 2048: 13 / 18 / 26 / 52 against 26 / 31 / 232 / 952 of ref_gemv_kernel
-    if (in % sm_kc(kSmW4) == 0 && g % 32 == 0 && in % g == 0 && out % 32 == 0 &&
+    if (in % sm_kc(kSmW4) == 0 && g % 32 == 0 && in % g == 0 && sm_out_ok(out) &&
         ((uintptr_t)qw & 3) == 0 && ((uintptr_t)x & 15) == 0) {
         SmArgs a{};
         a.x = x; a.w0 = qw; a.rb0 = in / 2; a.sc = sc; a.group = g; a.bias = bias; a.y = y;
@@ -203,7 +203,7 @@ int launch_ref_gemm_w4(const float* x, const uint8_t* qw, const float* sc, const
 int launch_ref_gemm_fp8(const float* x, const uint8_t* w, const float* sc, const float* bias,
                         float* y, int n, int in, int out, hipStream_t s) {
     // us at n = 1 / 8 / 64 / 203, 6144 -> 2048: 11 / 16 / 26 / 53 against 48 / 54 / 407 / 1498 of ref_gemv_kernel
-    if (in % sm_kc(kSmFp8) == 0 && out % 32 == 0 && ((uintptr_t)w & 3) == 0 &&
+    if (in % sm_kc(kSmFp8) == 0 && sm_out_ok(out) && ((uintptr_t)w & 3) == 0 &&
         ((uintptr_t)x & 15) == 0) {
         SmArgs a{};
         a.x = x; a.w0 = w; a.rb0 = in; a.sc = sc; a.group = in; a.bias = bias; a.y = y;

@@ -787,7 +787,7 @@ static bool gg_aligned(const void* w, long row_bytes, const void* x, int xalign)
 // weight rows and 16-byte aligned fp32 activations (int8: 4).
 static bool gg_sm_ok(uint32_t t, const void* w, long rb, const void* x, int xalign, int K, int out) {
     const bool type = t == 8 || t == 11 || t == 12 || t == 13 || t == 14 || t == 18 || t == 23;
-    return type && K % sm_kc(t) == 0 && out % 32 == 0 && gg_aligned(w, rb, x, xalign);
+    return type && K % sm_kc(t) == 0 && sm_out_ok(out) && gg_aligned(w, rb, x, xalign);
 }
 
 // f(constant) for a type gg_sm_ok accepts.

@@ -82,6 +82,9 @@ int sm_moe(bool down, bool i8, int tile, const SmArgs& a, unsigned tiles, hipStr
 template <uint32_t T>
 int sm_dense(bool i8, const SmArgs& a, hipStream_t s);
 
+// Output rows a launch takes: whole blocks of 32, in the grid's second dimension.
+constexpr bool sm_out_ok(int out) { return out % 32 == 0 && out / 32 <= 65535; }
+
 constexpr bool sm_g16(uint32_t t) { return t == 11 || t == 14; }          // scale per 16 K
 constexpr bool sm_min(uint32_t t) { return t == 12 || t == 13; }          // weight = ds * q - dm
 constexpr int sm_kc(uint32_t t) { return t == 8 || t == kSmFp8 ? 128 : 256; }   // K per chunk

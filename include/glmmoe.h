@@ -375,8 +375,10 @@ int glmmoe_ref_moe_expert_ffn(const float* x, const int* topk_ids, const float* 
 /* y[n, out] = x[n, in] . W[out, in]^T (+ bias), fp32 in and out, replacing
  * gemm_w4a16 (cuda/kernels.cuh:50-52, cuda/int4_gemm.cu:15-48): qW [out,
  * ceil(in/2)] u8, scales [out, ceil(in/group_size)] fp32, bias nullable; the
- * shared expert's linears. Any shape; in % 8 == 0 with group_size % 8 == 0
- * takes the staged path (a workgroup per 16 rows, tokens in blocks of 8). */
+ * shared expert's linears. Any shape; in % 256 == 0 with group_size % 32 == 0
+ * and out % 32 == 0 (x 16-byte, qW 4-byte aligned) runs on the matrix cores, fp32
+ * rows as three exact bf16 terms; in % 8 == 0 with group_size % 8 == 0 takes the
+ * staged vector path (a workgroup per 16 rows, tokens in blocks of 8). */
 int glmmoe_ref_gemm_w4a16(const float* x, const uint8_t* qW, const float* scales,
                           const float* bias, float* y, int64_t n, int64_t in, int64_t out,
                           int64_t group_size, void* stream);
@@ -407,7 +409,7 @@ int glmmoe_ref_add_inplace(float* y, const float* x, int64_t n, void* stream);
  * [n * topk, hidden] are caller scratch; out [n, hidden] is overwritten with
  * sum_s topk_w[t,s] * y_{t,s} in slot order. With `dispatch` (int scratch of
  * 3E + 1 + n*topk, nullable) the routed rows are grouped by expert first so
- * each weight row is read once per 8 rows of its expert; without it every
+ * each weight row is read once per 4 to 64 rows of its expert; without it every
  * routed row reads its expert's rows (the reference's token-major path).
  * gu_part (the reference's split-K partials) is accepted and not used.
  * Limits: every row length a multiple of its type's block and of 8,
