@@ -1206,18 +1206,18 @@ int launch_router_select(const uint16_t* x, const uint16_t* wr, const float* e_b
 // (round-to-nearest-even, as the bf16 entry's callers round them) on load,
 // then the same fixed order as the bf16 path: per 128-K chunk an ascending-K
 // fma chain from zero, chunk partials added in chunk order; then + bias[e]
-// (nullable). No workspace: grid (ceil(E / epw), ceil(n / 8)) of 512
+// (nullable). No workspace: grid (ceil(E / epw), ceil(n / 8)) of NTH
 // threads, thread (expert el, chunk c) for every token of its group of 8.
 // LDS: the group's activations as bf16 rows R = t * nchunks + c of 256 B,
 // 16-B piece o at slot o ^ (R & 15) (threads of consecutive chunks reading
 // the same piece hit distinct banks), then the partials [pair][token].
-constexpr int kF32Threads = 512;
 
 __host__ __device__ constexpr size_t f32_router_lds(int H, int epw) {
     return (size_t)kRouterTG * H * 2 + (size_t)epw * (H / kRouterKC) * kRouterTG * 4;
 }
 
-__global__ __launch_bounds__(kF32Threads) void router_logits_f32_kernel(
+template <int NTH>
+__global__ __launch_bounds__(NTH) void router_logits_f32_kernel(
     const float* __restrict__ x, const float* __restrict__ W, const float* __restrict__ bias,
     float* __restrict__ y, int n, int H, int E, int epw) {
     extern __shared__ __align__(16) char f32_lds[];
@@ -1228,7 +1228,7 @@ __global__ __launch_bounds__(kF32Threads) void router_logits_f32_kernel(
     float* part = reinterpret_cast<float*>(f32_lds + (size_t)kRouterTG * H * 2);
     // Stage: 8 consecutive K of one row per thread step (one 16-B piece).
     const int pieces = nt * (H / 8);
-    for (int i = tid; i < pieces; i += kF32Threads) {
+    for (int i = tid; i < pieces; i += NTH) {
         const int t = i / (H / 8), kp = i - t * (H / 8);
         const int c = kp / (kRouterKC / 8), o = kp % (kRouterKC / 8);
         const float4* src = reinterpret_cast<const float4*>(x + (size_t)(t0 + t) * H + kp * 8);
@@ -1278,8 +1278,8 @@ __global__ __launch_bounds__(kF32Threads) void router_logits_f32_kernel(
         }
     }
     __syncthreads();
-    if (tid < epw * kRouterTG) {
-        const int el2 = tid / kRouterTG, t = tid % kRouterTG;
+    for (int i = tid; i < epw * kRouterTG; i += NTH) {
+        const int el2 = i / kRouterTG, t = i % kRouterTG;
         const int e2 = blockIdx.x * epw + el2;
         if (e2 < E && t < nt) {
             const float total = chunk_sum(part + el2 * nchunks * kRouterTG + t, kRouterTG, nchunks);
@@ -1392,11 +1392,29 @@ __global__ __launch_bounds__(64 * NW) void router_f32_tiled_kernel(
     }
 }
 
+template <int NTH>
+static int go_router_f32(const float* x, const float* W, const float* bias, float* y, int n, int H, int E,
+                         hipStream_t s) {
+    static bool attr_set = false;
+    if (!attr_set) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&router_logits_f32_kernel<NTH>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)f32_router_lds(8192, NTH / (8192 / kRouterKC))) != hipSuccess)
+            return -4;
+        attr_set = true;
+    }
+    const int epw = NTH / (H / kRouterKC);
+    const dim3 grid((unsigned)((E + epw - 1) / epw), (unsigned)((n + kRouterTG - 1) / kRouterTG));
+    hipLaunchKernelGGL(router_logits_f32_kernel<NTH>, grid, dim3(NTH), f32_router_lds(H, epw), s, x, W, bias, y, n,
+                       H, E, epw);
+    return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
 int launch_router_logits_f32(const float* x, const float* W, const float* bias, float* y, int n,
                              int H, int E, hipStream_t s) {
-    if (H % kRouterKC || H / kRouterKC > kF32Threads || H > 8192) return -2;
+    if (H % kRouterKC || H > 8192) return -2;
     const int nchunks = H / kRouterKC;
-    const int epw = kF32Threads / nchunks;
+    const int epw = 512 / nchunks;
     const long blocks = (long)((E + epw - 1) / epw) * ((n + kRouterTG - 1) / kRouterTG);
     // The thread-per-chunk kernel holds up to one workgroup per CU (H 6144, E
     // 256: 64 tokens 28 us against 41 tiled, 96 tokens 52 against 41, 203: 80 /
@@ -1417,18 +1435,12 @@ int launch_router_logits_f32(const float* x, const float* W, const float* bias, 
                                H, E);
         return hipGetLastError() == hipSuccess ? 0 : -4;
     }
-    static bool attr_set = false;
-    if (!attr_set) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&router_logits_f32_kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)f32_router_lds(8192, kF32Threads / (8192 / kRouterKC))) != hipSuccess)
-            return -4;
-        attr_set = true;
-    }
-    dim3 grid((unsigned)((E + epw - 1) / epw), (unsigned)((n + kRouterTG - 1) / kRouterTG));
-    hipLaunchKernelGGL(router_logits_f32_kernel, grid, dim3(kF32Threads), f32_router_lds(H, epw), s, x, W,
-                       bias, y, n, H, E, epw);
-    return hipGetLastError() == hipSuccess ? 0 : -4;
+    // One token: the weights are the work, and workgroups of 128 threads put them
+    // on four times as many CUs (H 6144, E 256: 11.9 us to 11.1; H 2048: 11.3 to
+    // 9.1; H 4096, E 64: 12.1 to 10.0). From two tokens each workgroup's staging
+    // of the rows costs as much (H 6144, 2 tokens: 13.7 to 14.9).
+    if (n == 1) return go_router_f32<128>(x, W, bias, y, n, H, E, s);
+    return go_router_f32<512>(x, W, bias, y, n, H, E, s);
 }
 
 size_t router_logits_scratch_bytes(int n, int H, int E) {

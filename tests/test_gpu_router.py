@@ -139,10 +139,13 @@ def test_router_logits_f32_bit_exact(oracle):
         assert np.array_equal(yb.cpu().numpy().view(np.uint32), (ref + bias[None, :]).view(np.uint32)), (n, H, E)
 
 
-# The tiled kernel's launch shapes: one round of chunks with idle waves, several
-# rounds with a partial last one, ragged token and expert tiles.
-@pytest.mark.parametrize("n,H,E", [(9, 256, 16), (40, 1920, 33), (96, 6144, 256), (203, 8192, 100),
-                                   (1030, 384, 130), (1030, 2304, 130)])
+# The thread-per-chunk kernel's small workgroups (a partial last one, idle lanes,
+# more outputs than threads in either size). The tiled kernel's launch shapes: one
+# round of chunks with idle waves, several rounds with a partial last one, ragged
+# token and expert tiles.
+@pytest.mark.parametrize("n,H,E", [(1, 8192, 7), (2, 6144, 256), (2, 128, 300), (1, 128, 300),
+                                   (1, 1152, 65), (7, 256, 300), (9, 256, 16), (40, 1920, 33),
+                                   (96, 6144, 256), (203, 8192, 100), (1030, 384, 130), (1030, 2304, 130)])
 def test_router_logits_f32_tiled_bit_exact(oracle, n, H, E):
     rng = np.random.default_rng(n + H)
     x = rng.standard_normal((n, H)).astype(np.float32)
