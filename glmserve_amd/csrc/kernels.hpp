@@ -11,14 +11,7 @@ constexpr int kTileRows = 16;
 // Grouped rows per tile of the large-group (prefill) expert GEMMs.
 constexpr int kBigRows = 128;
 // Grouped rows (n*topk + n) from which the layer uses the large-group kernels.
-// The 16-row kernels stream each expert's weights once per 16 of its rows; at
-// uniform routing they stay ahead to about 11 rows per expert (6144 x 2048 x
-// 256, top-8, us, 16-row / 128-row kernels: 1152 rows 573 / 771, 2304 rows 780 /
-// 876, 2880 rows 887 / 912, 3600 rows 1028 / 956), with the rows on a few hot
-// experts (Zipf 1.1) to 1700 rows (1440: 270 / 295, 1710: 313 / 321, 1800: 341 /
-// 321, 2304: 421 / 323). The host does not know the skew: the line is where the
-// skewed batch breaks even.
-constexpr int kBigMinRows = 1664;
+constexpr int kBigMinRows = 1024;
 
 struct ExpertPtrs {
     const uint8_t* gate_q; const uint16_t* gate_s;

@@ -148,15 +148,15 @@ typedef struct glmmoe_layer_ws {
                              the expert's m full tiles, every batch size; 0 in the 4th
                              field for the 128-row layout's last tiles of 1-64 rows) */
     int* ntiles;          /* [3]: all tiles; the full tiles; the full and the 33-64-row
-                             tiles. The 128-row layout (from 1664 grouped rows) lists the
+                             tiles. The 128-row layout (from 1024 grouped rows) lists the
                              full tiles (more than 64 rows, or every tile of the 16-row
                              layout), then each expert's last tile of 33-64 rows, then of
                              1-32 rows; the 16-row layout has only full tiles */
     uint16_t* h;          /* [R, I] SiLU(gate) * up: bf16 (16-row tiles) or fp16 scaled
                              by 2^e per row (128-row tiles; e in hsum, below) */
-    float* hsum;          /* [R, I/128] group sums of h (decode kernels); from 1664 grouped rows
+    float* hsum;          /* [R, I/128] group sums of h (decode kernels); from 1024 grouped rows
                              the int8 exponents of h's 32-feature blocks, [R, I/32] bytes */
-    float* dpart;         /* [R, H] per-row expert outputs (unweighted): fp32 below 1664 grouped
+    float* dpart;         /* [R, H] per-row expert outputs (unweighted): fp32 below 1024 grouped
                              rows (n*topk + n), bf16 (first half of the region) from there;
                              at least 256 * (H / 2048) * 16 KiB: before the down projection
                              it holds the gate/up kernel's split-item partials */

@@ -252,14 +252,24 @@ def test_large_group_other_shape(oracle, n):
     _check_full(out, oracle_full_w4(L, oracle, x, ids, w))
 
 
-@pytest.mark.parametrize("n", [332, 333])
-def test_group_size_threshold(oracle, n):
-    # 1660 and 1665 grouped rows: the last batch of the 16-row kernels (experts
-    # of several tiles, routing of a large batch) and the first of the 128-row ones.
+@pytest.mark.parametrize("n,rows", [(204, 16), (205, 128)])
+def test_group_size_threshold(oracle, n, rows):
+    # 1020 and 1025 grouped rows: the last batch of the 16-row kernels and the
+    # first of the 128-row ones, which keep h in fp16 (11 significant bits
+    # against bf16's 8) and read an expert's weights once per 128 of its rows.
+    # The tile list says which ran.
     L = SynthLayer(1024, 8, 4, 1024, seed=10)
-    x, out, logits, ids, w, offs, st, sr = _run(L, n, seed=n)
-    ref_logits = _check_routing(oracle, L, x, logits, ids, w, offs, st, sr)
-    _check_full(out, oracle_full_w4(L, oracle, x, ids, w))
+    x = L.x(n, n)
+    ws = L.layer.alloc_workspace(n)
+    out = _nan_out(n, L.H)
+    L.layer.forward(x, out, ws)
+    torch.cuda.synchronize()
+    v = L.layer.workspace_view(n, ws)
+    ids = _ws_i32(ws, v.topk_ids, n * L.k).view(n, L.k).cpu().numpy()
+    w = _ws_f32(ws, v.topk_w, n * L.k).view(n, L.k).cpu().numpy()
+    counts = list(np.bincount(ids.reshape(-1), minlength=L.E)) + [n]   # the shared expert's rows
+    assert int(_ws_i32(ws, v.ntiles, 1)[0]) == sum(-(-int(c) // rows) for c in counts)
+    _check_full(out.cpu().numpy(), oracle_full_w4(L, oracle, x, ids, w))
 
 
 def test_split_last_round_deterministic():
