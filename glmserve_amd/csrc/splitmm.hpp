@@ -316,6 +316,26 @@ __device__ __forceinline__ sm_i32x2 sm_codes_i8(const uint8_t* b, int ib, int f,
     }
 }
 
+// Weights k .. k + 7 (k % 8 == 0) of a row (matrix row r), dequantized.
+template <uint32_t T>
+__device__ __forceinline__ void sm_weights(const SmArgs& a, const uint8_t* w, int r, int k, float (&y)[8]) {
+    if constexpr (T == kSmW4) {
+        const uint32_t c = gg_ld32(w + k / 2);
+        const float sc = a.sc[(size_t)r * (a.K / a.group) + k / a.group];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) y[u] = (float)((int)((c >> (4 * u)) & 15u) - 8) * sc;
+    } else if constexpr (T == kSmFp8) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int c = w[k + 2 * u] | w[k + 2 * u + 1] << 8;
+            const f32x2 p = __builtin_amdgcn_cvt_pk_f32_fp8(c, false);
+            y[2 * u] = p.x; y[2 * u + 1] = p.y;
+        }
+    } else {
+        gg_dec8<T>(T, w, k, c_iq3xxs_grid, y);
+    }
+}
+
 template <uint32_t T, bool I8, int RW, int KW, int NB, int NT, int KX>
 struct SmLds {
     static constexpr int XS = I8 ? KX + 16 : 2 * KX + 16;     // bytes of an activation row of a plane
@@ -515,21 +535,27 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
                 const uint32_t neg = (uint32_t)(s * BX + pc / 4) << 31;
 #pragma unroll
                 for (int u = 0; u < 8; ++u) v[u] = __uint_as_float(__float_as_uint(v[u]) ^ neg);
-                float m[8], l[8], chk = 0.0f;
+                float m[8], l[8];   // NaN for an infinity: the epilogue recomputes what is not finite
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
                     m[u] = v[u] - __uint_as_float(__float_as_uint(v[u]) & 0xffff0000u);
                     l[u] = m[u] - __uint_as_float(__float_as_uint(m[u]) & 0xffff0000u);
-                    chk += l[u];
                 }
-                if (chk != chk) {   // an infinity or NaN: its leading term alone
+                if constexpr (T == 8 && MODE != kSmDense) {
+                    // Clears what the epilogue recomputes anyway, for the branch's sake: without
+                    // it the compiler no longer mixes these kernels' decode with the products
+                    // (1024 x 512 x 8, top-2, 40 tokens: 47 -> 53 us).
+                    float chk = 0.0f;
 #pragma unroll
-                    for (int u = 0; u < 8; ++u)
-                        if (l[u] != l[u]) {
-                            m[u] = l[u] = 0.0f;
-                            // a NaN whose payload sits in the low half stays a NaN
-                            if (v[u] != v[u]) v[u] = __uint_as_float(0x7fc00000u);
-                        }
+                    for (int u = 0; u < 8; ++u) chk += l[u];
+                    if (chk != chk) {
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                            if (l[u] != l[u]) {
+                                m[u] = l[u] = 0.0f;
+                                if (v[u] != v[u]) v[u] = __uint_as_float(0x7fc00000u);
+                            }
+                    }
                 }
                 u32x4 ph, pm, pl;
 #pragma unroll
@@ -798,8 +824,11 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
             if constexpr (RW == 1) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             else sm_barrier();
             park_x(s);
+            // the order stays: split rows, next rows, next chunk
+            __builtin_amdgcn_sched_barrier(0);
             if (s + 1 < ST) load_x(cc * KC + (s + 1) * KX);
             else load_x(cn * KC);
+            __builtin_amdgcn_sched_barrier(0);
             // after the next step's activations: waiting for those (loads
             // complete in order) does not wait for the chunk
             if (s == 0) load_raw(cn);
@@ -888,6 +917,65 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
                 }
             }
         }
+
+    // Outputs that are not finite, from the dequantized weights instead: an infinite
+    // activation meets zeroed codes (16-K scales), a zero remainder term or the
+    // offset's sum as inf * 0 or inf - inf, and sums of codes overflow before their
+    // scale brings them back. A row of x at a time, lane = weight row and half of K.
+    if constexpr (!I8) {
+        uint32_t bad = 0;   // of the lane's values
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                float z = 0.0f;
+#pragma unroll
+                for (int nb = 0; nb < NK; ++nb) z = __builtin_fmaf(acc[nb][tb][i], 0.0f, z);
+                if (z != z) bad |= 1u << (tb * NV + i);
+            }
+        if (__builtin_expect(__ballot(bad != 0) != 0, 0)) {
+            __threadfence_block();   // the stores above come first
+            int ln = lane;
+            asm volatile("" : "+v"(ln));   // nothing of this is kept in registers through the main loop
+            const int half = ln >> 5;
+#pragma unroll 1
+            for (int t = 0; t < nr; ++t) {
+                const bool mine = SM ? t / NV == ln / 16 : ((t >> 2) & 1) == half;
+                const int v = SM ? t % NV : 16 * (t / 32) + 4 * (t % 32 / 8) + t % 4;
+                if (!__ballot(mine && (bad >> v & 1))) continue;
+                const float* xr = a.x + (size_t)L.src[t] * K;
+                float o[NB];
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) {
+                    const int r = ob[nb] + (ln & 31);
+                    const uint8_t* w = wb[nb] + (ln & 31) * rb[nb];
+                    double sum = 0.0;
+#pragma unroll 1
+                    for (int k = 8 * half; k < K; k += 16) {
+                        float y[8];
+                        sm_weights<T>(a, w, r, k, y);
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) sum = __builtin_fma((double)y[u], (double)xr[k + u], sum);
+                    }
+                    sum += __shfl_xor(sum, 32);
+                    if constexpr (T == kSmFp8) sum = a.sc ? sum * a.sc[r] : sum;
+                    o[nb] = (float)sum;
+                }
+                if (!half) {
+                    if constexpr (MODE == kSmGateUp) {
+                        if (f0 + 32 <= a.out)
+                            a.y[(size_t)L.row[t] * a.out + f0 + ln] = o[0] / (1.0f + expf(-o[0])) * o[1];
+                    } else {
+                        float* y = a.y + (MODE == kSmDown ? (size_t)L.row[t] : (size_t)(t0 + t)) * a.out + f0 + ln;
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb)
+                            if (f0 + 32 * nb + 32 <= a.out)
+                                y[32 * nb] = MODE == kSmDense && a.bias ? o[nb] + a.bias[f0 + 32 * nb + ln] : o[nb];
+                    }
+                }
+            }
+        }
+    }
 }
 
 }  // namespace glmmoe

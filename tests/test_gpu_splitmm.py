@@ -156,30 +156,117 @@ def test_moe(oracle, types, n, grouped):
     assert _err(out.cpu().numpy(), ref_out(hd.reshape(n * k, I))) < tol
 
 
-@pytest.mark.parametrize("qtype", [8, 18])
-def test_extreme_activations(oracle, qtype):
-    # Tokens of very large and very small rows keep their relative accuracy; an
-    # infinity or NaN stays in its token and gives what the fp32 product gives.
-    rng = np.random.default_rng(3 + qtype)
-    n, in_, out = 6, 512, 64
+def _extreme_rows(in_, W, rng):
+    """Rows of ordinary, very large and very small magnitudes, then one with an
+    infinity and one with a NaN. The largest has outputs near the top of fp32 (its
+    sums of codes alone overflow)."""
+    x = rng.standard_normal((8, in_)).astype(np.float32)
+    x[1] *= np.float32(1e30 if np.abs(W).max() < 1e3 else 1e25)
+    x[2] *= np.float32(1e-25)
+    x[3, ::2] *= np.float32(1e-6)   # small terms beside large ones
+    x[4] *= np.float32(1e37 / np.abs(x[4].astype(np.float64) @ W.T).max())
+    x[6, 77] = -np.inf
+    x[7, 200] = np.nan
+    return x
+
+
+def _check_extreme(got, x, W, tol):
+    # Every row's relative accuracy; an infinity or NaN stays in its row and gives
+    # what the product with the dequantized weights gives (NaN for a zero weight).
+    ref = x.astype(np.float64) @ W.T
+    for t in range(6):
+        assert _err(got[t], ref[t]) < tol, t   # a norm over few outputs only: twice the bound
+    with np.errstate(invalid="ignore"):
+        inf = np.float32(-np.inf) * W[:, 77].astype(np.float32)
+    assert np.array_equal(got[6], inf, equal_nan=True)
+    assert np.isnan(got[7]).all()
+
+
+# The tiles of 4 (a row at a time), 16 and 32 tokens.
+@pytest.mark.parametrize("fmt", TYPES + ["w4", "fp8"])
+def test_extreme_activations(oracle, fmt):
+    in_, out = 512, 64
+    rng = np.random.default_rng(TYPES.index(fmt) if fmt in TYPES else len(fmt))
+    if fmt == "w4":
+        q = rng.integers(0, 256, (out, in_ // 2), dtype=np.uint8)
+        s = rng.uniform(0.001, 0.02, (out, in_ // 128)).astype(np.float32)
+        W = oracle.dequant_int4_rows(q, s, in_, 128).astype(np.float64)
+        run = lambda x, y: ops.ref_gemm_w4a16(x, _dev(q), _dev(s), None, y, 128)
+    elif fmt == "fp8":
+        c = rng.integers(0, 256, (out, in_), dtype=np.uint8)
+        c[(c & 0x7F) == 0x7F] = 0x3C
+        sc = rng.uniform(0.5e-3, 1.5e-3, out).astype(np.float32)
+        W = np.array([oracle.e4m3_to_f32(v) for v in range(256)], np.float64)[c] * sc[:, None].astype(np.float64)
+        run = lambda x, y: ops.ref_gemm_fp8(x, _dev(c), _dev(sc), None, y)
+    else:
+        w = random_gguf_rows(fmt, out, in_, rng)
+        W = oracle.gguf_dequant_rows(fmt, w, out, in_).astype(np.float64)
+        run = lambda x, y: ops.ref_gemm_q(fmt, x, _dev(w), None, y, w.shape[1])
+    x = _extreme_rows(in_, W, rng)
+    tol = 2 * TOL.get(fmt, 2.5e-7)
+    for reps in (1, 3):
+        y = torch.zeros(8 * reps, out, device="cuda")
+        run(_dev(np.tile(x, (reps, 1))), y)
+        for r in range(reps):
+            _check_extreme(y.cpu().numpy()[8 * r:8 * r + 8], x, W, tol)
+    y = torch.zeros(8, out, device="cuda")
+    for t in range(8):
+        run(_dev(x[t:t + 1]), y[t:t + 1])
+    _check_extreme(y.cpu().numpy(), x, W, tol)
+
+
+@pytest.mark.parametrize("qtype", [8, 12, 18])
+def test_extreme_activations_large_tiles(oracle, qtype):
+    rng = np.random.default_rng(qtype)
+    n, in_, out = 385, 256, 7168 - 32
     w = random_gguf_rows(qtype, out, in_, rng)
     W = oracle.gguf_dequant_rows(qtype, w, out, in_).astype(np.float64)
     x = rng.standard_normal((n, in_)).astype(np.float32)
-    x[1] *= np.float32(1e30)
-    x[2] *= np.float32(1e-25)
-    x[3, ::2] *= np.float32(1e-6)   # small terms beside large ones
-    x[4, 77] = -np.inf
-    x[5, 300] = np.nan
+    ext = _extreme_rows(in_, W, rng)
+    x[60:68] = ext
+    x[384] = ext[4]
     y = torch.zeros(n, out, device="cuda")
-    ops.ref_gemm_q(qtype, _dev(x), _dev(w), None, y, w.shape[1])
+    wp = np.concatenate([w, np.zeros((out, -w.shape[1] % 4), np.uint8)], 1)
+    ops.ref_gemm_q(qtype, _dev(x), _dev(wp), None, y, wp.shape[1])
     got = y.cpu().numpy()
-    ref = x[:4].astype(np.float64) @ W.T
-    for t in range(4):
-        assert _err(got[t], ref[t]) < 5e-7, t   # a norm over 64 outputs only
-    with np.errstate(invalid="ignore"):
-        inf = np.float32(-np.inf) * W[:, 77].astype(np.float32)   # NaN for a zero weight
-    assert np.array_equal(got[4], inf, equal_nan=True)
-    assert np.isnan(got[5]).all()
+    _check_extreme(got[60:68], ext, W, 2 * TOL[qtype])
+    ok = np.r_[0:60, 68:385]
+    assert _err(got[ok], x[ok].astype(np.float64) @ W.T) < TOL[qtype]
+
+
+# Tiles of 4 (ungrouped), 8 or 16, and 32 rows: gate and up of a token with an infinity,
+# and of one whose sums of codes overflow.
+@pytest.mark.parametrize("types", [(18, 18, 23), (12, 12, 14), (14, 14, 8)])
+@pytest.mark.parametrize("n,grouped", [(3, False), (9, True), (70, True)])
+def test_moe_extreme_activations(oracle, types, n, grouped):
+    H, I, E, k = 1024, 512, 8, 4
+    rng = np.random.default_rng(sum(types) + n)
+    geo = [(types[0], I, H), (types[1], I, H), (types[2], H, I)]
+    pk = [_rows(t, E * r, c, rng) for t, r, c in geo]
+    W = [oracle.gguf_dequant_rows(t, p[1], E * r, c).reshape(E, r, c).astype(np.float64)
+         for (t, r, c), p in zip(geo, pk)]
+    x = (rng.standard_normal((n, H)) * 2e-2).astype(np.float32)
+    x[1, 5] = np.inf
+    ids = np.stack([rng.permutation(E)[:k] for _ in range(n)]).astype(np.int32)
+    x[2] *= np.float32(1e18 / np.abs(np.einsum("k,erk->er", x[2].astype(np.float64), W[1])).max())
+    w = rng.uniform(0.1, 1.0, (n, k)).astype(np.float32)
+    f = lambda *s: torch.zeros(*s, device="cuda")
+    h_act, dpart, out = f(n * k, I), f(n * k, H), f(n, H)
+    disp = torch.zeros(3 * E + 1 + n * k, dtype=torch.int32, device="cuda") if grouped else None
+    ops.ref_moe_expert_ffn_q(types, _dev(x), _dev(ids), _dev(w), *[_dev(p[0]) for p in pk], I, E,
+                             tuple(p[0].shape[1] for p in pk), h_act, dpart, out, disp)
+    h, d = h_act.cpu().numpy(), dpart.cpu().numpy()
+    tol = 4 * max(TOL[t] for t in types)
+    for r in range(n * k):
+        t, e = r // k, ids[r // k, r % k]
+        with np.errstate(invalid="ignore", over="ignore"):
+            g, u = ((np.inf * W[m][e][:, 5] if t == 1 else W[m][e] @ x[t].astype(np.float64)) for m in (0, 1))
+            ref = (g / (1 + np.exp(-g)) * u).astype(np.float32)
+        if t == 1:
+            assert np.array_equal(h[r], ref, equal_nan=True)
+            continue
+        assert _err(h[r].astype(np.float64), ref) < tol and np.isfinite(d[r]).all()
+        assert _err(d[r].astype(np.float64), W[2][e] @ h[r].astype(np.float64)) < tol
 
 
 def test_unaligned_elementwise(oracle):
