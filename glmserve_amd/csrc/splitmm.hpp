@@ -6,9 +6,9 @@
 // int8 for the GGUF types), so the codes are the MFMA's B operand as they are
 // and the scale multiplies the 16- or 32-K partial product afterwards, in
 // fp32, once per output.
-// fp32 activations are cut into three bf16 terms by truncation (8 + 8 + 8
-// significant bits: the three add up to the fp32 value exactly), three MFMAs
-// per 16 K, smallest term first. Products are exact, the MFMA adds in fp32:
+// fp32 activations, times 2^40, are cut into three bf16 terms by truncation (8 +
+// 8 + 8 significant bits: the three add up to the fp32 value exactly), three
+// MFMAs per 16 K, smallest term first. Products are exact, the MFMA adds in fp32:
 // the rounding is that of an fp32 sum over 16- or 32-K pieces.
 // int8 activations use the int8 MFMA (exact int32 sums per 32 K), then the
 // weight scale and the activation block's scale in fp32.
@@ -81,6 +81,11 @@ template <uint32_t T>
 int sm_moe(bool down, bool i8, int tile, const SmArgs& a, unsigned tiles, hipStream_t s);
 template <uint32_t T>
 int sm_dense(bool i8, const SmArgs& a, hipStream_t s);
+
+// fp32 activations are split times 2^40: the matrix cores take subnormal bf16 terms
+// as zero, and an activation below 2^-110 has some (rows of about 1e-36 lost three
+// digits). From 2^88 the epilogue recomputes.
+constexpr float kSmUp = 0x1p40f;
 
 // Output rows a launch takes: whole blocks of 32, in the grid's second dimension.
 constexpr bool sm_out_ok(int out) { return out % 32 == 0 && out / 32 <= 65535; }
@@ -529,12 +534,12 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
                     float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
                     sum += __shfl_xor(sum, 1);
                     sum += __shfl_xor(sum, 2);
-                    if (!(pc & 3)) L.xsum[kw][pc / 4][t] = sum;
+                    if (!(pc & 3)) L.xsum[kw][pc / 4][t] = sum * kSmUp;
                 }
                 // odd 32-K blocks enter negated (see the head of the file)
-                const uint32_t neg = (uint32_t)(s * BX + pc / 4) << 31;
+                const float up = (s * BX + pc / 4) & 1 ? -kSmUp : kSmUp;
 #pragma unroll
-                for (int u = 0; u < 8; ++u) v[u] = __uint_as_float(__float_as_uint(v[u]) ^ neg);
+                for (int u = 0; u < 8; ++u) v[u] *= up;
                 float m[8], l[8];   // NaN for an infinity: the epilogue recomputes what is not finite
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
@@ -887,6 +892,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
     }
 
     // Stores: BR lanes write BR consecutive outputs of a token.
+    constexpr Acc kOut = I8 ? 1.0f : 1.0f / kSmUp;
 #pragma unroll
     for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
@@ -897,7 +903,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
                 if (f0 + 32 > a.out) continue;
 #pragma unroll
                 for (int nb = 0; nb < NK / 2; ++nb) {
-                    const Acc g = acc[nb][tb][i], u = acc[nb + NK / 2][tb][i];
+                    const Acc g = acc[nb][tb][i] * kOut, u = acc[nb + NK / 2][tb][i] * kOut;
                     float& h = a.y[(size_t)L.row[t] * a.out + f0 + nb * BR + lr];
                     if constexpr (F64) h = (float)(g / (1.0 + exp(-g)) * u);
                     else h = g / (1.0f + expf(-g)) * u;
@@ -908,7 +914,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
                 for (int nb = 0; nb < NK; ++nb) {
                     const int o = f0 + nb * BR;
                     if (f0 + 32 * (nb * BR / 32) + 32 > a.out) continue;
-                    float v = (float)acc[nb][tb][i];
+                    float v = (float)(acc[nb][tb][i] * kOut);
                     if constexpr (MODE == kSmDense) {
                         if constexpr (T == kSmFp8) v = a.sc ? v * a.sc[o + lr] : v;
                         if (a.bias) v += a.bias[o + lr];

@@ -159,12 +159,13 @@ def test_moe(oracle, types, n, grouped):
 def _extreme_rows(in_, W, rng):
     """Rows of ordinary, very large and very small magnitudes, then one with an
     infinity and one with a NaN. The largest has outputs near the top of fp32 (its
-    sums of codes alone overflow)."""
+    sums of codes alone overflow), the smallest subnormal low-order terms."""
     x = rng.standard_normal((8, in_)).astype(np.float32)
     x[1] *= np.float32(1e30 if np.abs(W).max() < 1e3 else 1e25)
     x[2] *= np.float32(1e-25)
     x[3, ::2] *= np.float32(1e-6)   # small terms beside large ones
     x[4] *= np.float32(1e37 / np.abs(x[4].astype(np.float64) @ W.T).max())
+    x[5] *= np.float32(1e-36)
     x[6, 77] = -np.inf
     x[7, 200] = np.nan
     return x
