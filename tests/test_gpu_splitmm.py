@@ -270,6 +270,25 @@ def test_moe_extreme_activations(oracle, types, n, grouped):
         assert _err(d[r].astype(np.float64), W[2][e] @ h[r].astype(np.float64)) < tol
 
 
+# Q4_K / Q5_K weights centred on zero (as a checkpoint's are) with activations off zero: the
+# offsets' sum must not take the product's accuracy with it.
+@pytest.mark.parametrize("qtype", [12, 13])
+@pytest.mark.parametrize("n", [3, 9, 40])
+def test_offset_activations(oracle, qtype, n):
+    rng = np.random.default_rng(qtype + n)
+    in_, out = 6144, 512
+    w = random_gguf_rows(qtype, out, in_, rng)
+    b = w.reshape(out, in_ // 256, -1)
+    d = np.ascontiguousarray(b[:, :, 0:2]).view(np.float16).astype(np.float32)
+    b[:, :, 2:4] = (d * (7.5 if qtype == 12 else 15.5)).astype(np.float16).view(np.uint8)
+    W = oracle.gguf_dequant_rows(qtype, w, out, in_).astype(np.float64)
+    x = (rng.standard_normal((n, in_)) + 1).astype(np.float32)
+    y = torch.zeros(n, out, device="cuda")
+    ops.ref_gemm_q(qtype, _dev(x), _dev(w), None, y, w.shape[1])
+    # the types without an offset have 9.5e-8 here at most; 10 % for the two roundings more per block
+    assert _err(y.cpu().numpy(), x.astype(np.float64) @ W.T) < 1.045e-7
+
+
 def test_unaligned_elementwise(oracle):
     # quantize_act_q8 and the combine on rows that are not 16-byte aligned.
     rng = np.random.default_rng(8)
