@@ -363,8 +363,9 @@ struct SmLds {
     int src[NT], row[NT], tile[3];
     // from here on free for the shares' sums at the end
     __align__(16) uint8_t x[KW][PL][NT][XS];
-    float xsc[I8 ? KW : 1][I8 ? KX / 32 : 1][I8 ? NT : 1];               // int8 block scales
-    float xsum[sm_min(T) ? KW : 1][sm_min(T) ? KX / 32 : 1][sm_min(T) ? NT : 1];   // block sums
+    // read as float4 in the tiles of 32 and 64: rows of NT floats from 16-byte aligned starts
+    __align__(16) float xsc[I8 ? KW : 1][I8 ? KX / 32 : 1][I8 ? NT : 1];           // int8 block scales
+    __align__(16) float xsum[sm_min(T) ? KW : 1][sm_min(T) ? KX / 32 : 1][sm_min(T) ? NT : 1];   // block sums
     float ds[RW * KW][NB * 32][NS + 1];
     float dm[sm_min(T) ? RW * KW : 1][sm_min(T) ? NB * 32 : 1][NS + 1];
     __align__(16) uint8_t raw[RW * KW][NB * 32][sm_stride(T)];
@@ -375,6 +376,7 @@ template <uint32_t T, int MODE, bool I8, int RW, int KW, int NB, int NT, int KX>
 __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
     using S = SmLds<T, I8, RW, KW, NB, NT, KX>;
     static_assert(MODE != kSmGateUp || NB == 2, "gate and up rows in one wave");
+    static_assert(offsetof(S, xsc) % 16 == 0 && offsetof(S, xsum) % 16 == 0 && NT % 4 == 0, "float4 reads");
     constexpr bool SM = NT <= 16;                 // 16x16x32 MFMAs
     constexpr int TOK = NT, KC = sm_kc(T), ST = KC / KX, BX = KX / 32;
     constexpr int TB = SM ? 1 : NT / 32;          // 32-token blocks
