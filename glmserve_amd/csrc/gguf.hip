@@ -937,12 +937,12 @@ static int gg_sm_tile(const GgMoeArgs& a, bool grouped) {
     if (nk <= 4 * E) return 8;
     if (I8 && nk < 2048) return 16;
     auto kquant = [](uint32_t t) { return t >= 11 && t <= 14; };
+    const bool large = sm_large_tile(gt, I8) && sm_large_tile(dt, I8);
     if (kquant(gt) || kquant(dt)) {
         const bool long16 = (sm_g16(gt) && a.H > 4096) || (sm_g16(dt) && a.I > 4096);
         return nk <= 16 * E || long16 ? 16 : kSmMidTile;
     }
-    if (I8) return nk <= 16 * E ? kSmMidTile : kSmLargeTile;
-    return nk <= 64 * E || gt == 8 || dt == 8 ? kSmMidTile : kSmLargeTile;
+    return nk <= (I8 ? 16 : 64) * E || !large ? kSmMidTile : kSmLargeTile;
 }
 
 // Gate/up and down on splitmm_kernel; d: the grouping in tiles of `tile` rows.

@@ -76,7 +76,10 @@ struct SmArgs {
 
 // Tokens per tile of the large MoE launches; the small ones take 4, 8 or 16.
 constexpr int kSmMidTile = 32, kSmLargeTile = 64;
-// The launches (splitmm_launch.hpp): tile = tokens per tile of the grouping.
+// The types whose experts take tiles of 64 (the measurements: gg_sm_tile).
+constexpr bool sm_large_tile(uint32_t t, bool i8) { return t == 18 || t == 23 || (t == 8 && i8); }
+// The launches (splitmm_launch.hpp): tile = tokens per tile of the grouping; a tile
+// the type has no kernel for is refused (-2).
 template <uint32_t T>
 int sm_moe(bool down, bool i8, int tile, const SmArgs& a, unsigned tiles, hipStream_t s);
 template <uint32_t T>

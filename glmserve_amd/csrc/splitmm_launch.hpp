@@ -16,23 +16,26 @@ static int sm_go(const SmArgs& a, unsigned gx, hipStream_t s) {
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
-// K staged at a time for tiles of nt tokens; less where a row's chunk is wide,
-// so that two workgroups' LDS fits a CU.
+// K staged at a time for tiles of nt tokens; less where a row's chunk is wide, so
+// that two workgroups' LDS fits a CU (all but the 8- and 16-token expert tiles of
+// Q6_K with fp32 rows: 84 and 85 KiB).
 constexpr int sm_kx(uint32_t t, int nt) {
     const int k = nt <= 8 ? 128 : 64;
     return t == 12 || t == 13 || t == 14 ? k / 2 : k;
 }
 
+// -2: a tile that no call of this type takes (sm_large_tile).
 template <uint32_t T, int MODE, bool I8>
 static int sm_moe_mode(int tile, const SmArgs& a, unsigned tiles, hipStream_t s) {
     if (tile == 4) return sm_go<T, MODE, I8, 1, 4, 2, 4, sm_kx(T, 4)>(a, tiles, s);
     if (tile == 8) return sm_go<T, MODE, I8, 1, 4, 2, 8, sm_kx(T, 8)>(a, tiles, s);
+    if (tile == 16) return sm_go<T, MODE, I8, 1, 4, 2, 16, sm_kx(T, 16)>(a, tiles, s);
     if (tile == kSmMidTile)
         return sm_go<T, MODE, I8, 4, 1, 2, 32, I8 || T == 8 ? 128 : T == 14 ? 32 : 64>(a, tiles, s);
-    if constexpr (!sm_g16(T)) {
+    if constexpr (sm_large_tile(T, I8)) {
         if (tile == kSmLargeTile) return sm_go<T, MODE, I8, 4, 1, 2, 64, I8 ? 128 : sm_kx(T, 64)>(a, tiles, s);
     }
-    return sm_go<T, MODE, I8, 1, 4, 2, 16, sm_kx(T, 16)>(a, tiles, s);
+    return -2;
 }
 
 template <uint32_t T>

@@ -305,3 +305,18 @@ def test_fp8_host_checks_and_workspace():
         assert v.xscale - v.xq >= n * 6144 and v.hscale - v.hq >= R * 2048
         assert v.dpart + R * 6144 * 4 <= base + b
     assert L.glmmoe_moe_layer_fp8(C.byref(st), dummy, 4, dummy, dummy, 16, None) == -3
+
+
+@pytest.mark.parametrize("qtype", [8, 11, 12, 13, 14, 18, 23])
+def test_expert_tiles_without_a_kernel_are_refused(qtype):
+    # The matrix-core experts' launcher under its C++ name: a tile size the type has
+    # no kernel for must not run another tile's kernel on that grouping (64-row tiles
+    # in steps of 16 would leave rows uncomputed). Refused before any HIP call.
+    f = getattr(_lib.lib(), f"_ZN6glmmoe6sm_moeILj{qtype}EEEibbiRKNS_6SmArgsEjP12ihipStream_t")
+    f.argtypes = [C.c_bool, C.c_bool, C.c_int, C.c_void_p, C.c_uint, C.c_void_p]
+    args = (C.c_char * 512)()   # never read
+    for down in (False, True):
+        for i8 in (False, True):
+            large = qtype in (18, 23) or (qtype == 8 and i8)
+            for tile in [0, 1, 24, 128] + ([] if large else [64]):
+                assert f(down, i8, tile, C.cast(args, C.c_void_p), 1, None) == -2, (down, i8, tile)
