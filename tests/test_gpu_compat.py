@@ -85,6 +85,23 @@ def test_ref_silu_mul_and_add_inplace():
     assert torch.equal(yd.cpu(), y + u)
 
 
+# Four elements per thread where all rows are 16-byte aligned, else one; the last
+# n % 4 by themselves, nothing written behind them.
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 1024, 1030])
+@pytest.mark.parametrize("off", [(0, 0, 0), (1, 0, 0), (0, 0, 3)])
+def test_ref_silu_mul_edges(n, off):
+    gen = _gen(n)
+    g, u, out = [torch.full((n + 8,), 7.0, device="cuda")[o:] for o in off]
+    gh, uh = torch.randn(n, generator=gen) * 8, torch.randn(n, generator=gen)
+    g[:n], u[:n] = gh.cuda(), uh.cuda()
+    ops.ref_silu_mul(g[:n], u[:n], out[:n])
+    ref = gh.double() / (1 + torch.exp(-gh.double())) * uh.double()
+    got = out.cpu()
+    # the 64-bit value rounded once: half an ulp, and the last bits of exp
+    assert torch.allclose(got[:n].double(), ref, rtol=2.0 ** -24 * 1.001, atol=1e-45)
+    assert (got[n:] == 7.0).all()
+
+
 def _routing(oracle, n, E, k, seed):
     gen = np.random.default_rng(seed)
     logits = gen.standard_normal((n, E)).astype(np.float32)
