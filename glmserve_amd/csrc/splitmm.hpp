@@ -912,6 +912,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
 
     // Stores: BR lanes write BR consecutive outputs of a token.
     constexpr Acc kOut = I8 ? 1.0f : 1.0f / kSmUp;
+    float z = 0.0f;   // NaN once one of the lane's sums is not finite
 #pragma unroll
     for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
@@ -923,6 +924,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
 #pragma unroll
                 for (int nb = 0; nb < NK / 2; ++nb) {
                     const Acc g = acc[nb][tb][i] * kOut, u = acc[nb + NK / 2][tb][i] * kOut;
+                    if constexpr (!I8) z = __builtin_fmaf(g, 0.0f, __builtin_fmaf(u, 0.0f, z));
                     float& h = a.y[(size_t)L.row[t] * a.out + f0 + nb * BR + lr];
                     if constexpr (F64) h = (float)(g / (1.0 + exp(-g)) * u);
                     else h = g / (1.0f + expf(-g)) * u;
@@ -934,6 +936,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
                     const int o = f0 + nb * BR;
                     if (f0 + 32 * (nb * BR / 32) + 32 > a.out) continue;
                     float v = (float)(acc[nb][tb][i] * kOut);
+                    if constexpr (!I8) z = __builtin_fmaf(v, 0.0f, z);
                     if constexpr (MODE == kSmDense) {
                         if constexpr (T == kSmFp8) v = a.sc ? v * a.sc[o + lr] : v;
                         if (a.bias) v += a.bias[o + lr];
@@ -946,28 +949,26 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
     // Outputs that are not finite, from the dequantized weights instead: an infinite
     // activation meets zeroed codes (16-K scales), a zero remainder term or the
     // offset's sum as inf * 0 or inf - inf, and sums of codes overflow before their
-    // scale brings them back. A row of x at a time, lane = weight row and half of K.
+    // scale brings them back. The rows concerned are found among the stored outputs
+    // (a sum that is not finite gives no finite output): one register through the
+    // stores. With the sums themselves kept for it the compiler spilled in the main
+    // loop (Q4_K experts, 2048 x 512 x 64, top-4, 1000 tokens: 282 -> 343 us).
+    // A row of x at a time, lane = weight row and half of K.
     if constexpr (!I8) {
-        uint32_t bad = 0;   // of the lane's values
-#pragma unroll
-        for (int tb = 0; tb < TB; ++tb)
-#pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                float z = 0.0f;
-#pragma unroll
-                for (int nb = 0; nb < NK; ++nb) z = __builtin_fmaf(acc[nb][tb][i], 0.0f, z);
-                if (z != z) bad |= 1u << (tb * NV + i);
-            }
-        if (__builtin_expect(__ballot(bad != 0) != 0, 0)) {
+        if (__builtin_expect(__ballot(z != z) != 0, 0)) {
             __threadfence_block();   // the stores above come first
             int ln = lane;
             asm volatile("" : "+v"(ln));   // nothing of this is kept in registers through the main loop
             const int half = ln >> 5;
+            constexpr int NY = MODE == kSmGateUp ? 1 : NB;   // output blocks
 #pragma unroll 1
             for (int t = 0; t < nr; ++t) {
-                const bool mine = SM ? t / NV == ln / 16 : ((t >> 2) & 1) == half;
-                const int v = SM ? t % NV : 16 * (t / 32) + 4 * (t % 32 / 8) + t % 4;
-                if (!__ballot(mine && (bad >> v & 1))) continue;
+                float* y = a.y + (MODE == kSmDense ? (size_t)(t0 + t) : (size_t)L.row[t]) * a.out + f0 + (ln & 31);
+                float zt = 0.0f;
+#pragma unroll
+                for (int nb = 0; nb < NY; ++nb)
+                    if (f0 + 32 * nb + 32 <= a.out) zt = __builtin_fmaf(y[32 * nb], 0.0f, zt);
+                if (!__ballot(zt != zt)) continue;
                 const float* xr = a.x + (size_t)L.src[t] * K;
                 float o[NB];
 #pragma unroll
@@ -977,26 +978,21 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
                     double sum = 0.0;
 #pragma unroll 1
                     for (int k = 8 * half; k < K; k += 16) {
-                        float y[8];
-                        sm_weights<T>(a, w, r, k, y);
+                        float v[8];
+                        sm_weights<T>(a, w, r, k, v);
 #pragma unroll
-                        for (int u = 0; u < 8; ++u) sum = __builtin_fma((double)y[u], (double)xr[k + u], sum);
+                        for (int u = 0; u < 8; ++u) sum = __builtin_fma((double)v[u], (double)xr[k + u], sum);
                     }
                     sum += __shfl_xor(sum, 32);
                     if constexpr (T == kSmFp8) sum = a.sc ? sum * a.sc[r] : sum;
                     o[nb] = (float)sum;
                 }
+                if constexpr (MODE == kSmGateUp) o[0] = o[0] / (1.0f + expf(-o[0])) * o[1];
                 if (!half) {
-                    if constexpr (MODE == kSmGateUp) {
-                        if (f0 + 32 <= a.out)
-                            a.y[(size_t)L.row[t] * a.out + f0 + ln] = o[0] / (1.0f + expf(-o[0])) * o[1];
-                    } else {
-                        float* y = a.y + (MODE == kSmDown ? (size_t)L.row[t] : (size_t)(t0 + t)) * a.out + f0 + ln;
 #pragma unroll
-                        for (int nb = 0; nb < NB; ++nb)
-                            if (f0 + 32 * nb + 32 <= a.out)
-                                y[32 * nb] = MODE == kSmDense && a.bias ? o[nb] + a.bias[f0 + 32 * nb + ln] : o[nb];
-                    }
+                    for (int nb = 0; nb < NY; ++nb)
+                        if (f0 + 32 * nb + 32 <= a.out)
+                            y[32 * nb] = MODE == kSmDense && a.bias ? o[nb] + a.bias[f0 + 32 * nb + ln] : o[nb];
                 }
             }
         }
