@@ -174,8 +174,11 @@ def test_gemm_q_i8_unaligned_rows(oracle):
     assert rel_err(y.cpu().numpy(), ref) < 1e-5
 
 
-@pytest.mark.parametrize("types", [(18, 18, 23), (8, 8, 8), (23, 23, 18)])
-def test_moe_expert_ffn_q_i8_matrix_cores(oracle, types):
+# pad: zero bytes behind each down row. Packed, IQ3_XXS rows of one block are 98 bytes,
+# no whole dwords: both phases then stay on the vector kernels.
+@pytest.mark.parametrize("types,pad", [((18, 18, 23), 0), ((8, 8, 8), 0), ((23, 23, 18), 0),
+                                       ((23, 23, 18), 2)])
+def test_moe_expert_ffn_q_i8_matrix_cores(oracle, types, pad):
     # n * topk = 2048 routed rows with the grouping scratch: the matrix-core
     # phases (v_mfma_i32_32x32x32_i8 per 32-block, then the fp32 rescale; the
     # reference's tensor-core policy, cuda/qgemm.cu:1563-1587) on the types
@@ -183,14 +186,15 @@ def test_moe_expert_ffn_q_i8_matrix_cores(oracle, types):
     # h_act against the oracle's fp64 sums of the same integer products
     # (1e-5), (hq, hs) bit for bit against the oracle's quantizer of that
     # h_act, out against the oracle's int8 down and slot-order combine (1e-5);
-    # then the fp32 layer within 3e-2, and the token-major run (no grouping:
-    # the VALU kernels): h_act within 1e-5, the output within 1e-2 (after the
+    # then the fp32 layer within 3e-2, and the token-major run (no grouping: tiles
+    # of one row): h_act within 1e-5, the output within 1e-2 (after the
     # requantization of h, see below).
     H, I, E, k, n = 512, 256, 8, 4, 512
     rng = np.random.default_rng(sum(types) + 123)
     gq = random_gguf_rows(types[0], E * I, H, rng)
     uq = random_gguf_rows(types[1], E * I, H, rng)
     dq = random_gguf_rows(types[2], E * H, I, rng)
+    dqp = np.concatenate([dq, np.zeros((E * H, pad), np.uint8)], 1)
     rb = (_row_bytes(types[0], H), _row_bytes(types[1], H), _row_bytes(types[2], I))
     x = rng.standard_normal((n, H)).astype(np.float32)
     ids = np.stack([rng.permutation(E)[:k] for _ in range(n)]).astype(np.int32)
@@ -210,7 +214,7 @@ def test_moe_expert_ffn_q_i8_matrix_cores(oracle, types):
         disp = (torch.full((3 * E + 1 + n * k,), -7, dtype=torch.int32, device="cuda")
                 if grouped else None)
         ops.ref_moe_expert_ffn_q_i8(types, xq, xs, _dev(ids), _dev(w), _dev(gq), _dev(uq),
-                                    _dev(dq), I, E, rb, h_act, hq, hs, dpart, out, disp)
+                                    _dev(dqp), I, E, (*rb[:2], rb[2] + pad), h_act, hq, hs, dpart, out, disp)
         torch.cuda.synchronize()
         outs.append((h_act.cpu().numpy(), hq.cpu().numpy(), hs.cpu().numpy(),
                      out.cpu().numpy()))

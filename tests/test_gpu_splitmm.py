@@ -27,7 +27,9 @@ def _dev(a):
 
 
 def _rows(t, rows, k, rng):
-    """GGUF rows with row_bytes rounded up to a multiple of 4 (dword-aligned rows)."""
+    """GGUF rows with row_bytes rounded up to a multiple of 4, and as packed. The matrix
+    cores take whole dwords: an odd number of 98-, 110- or 210-byte blocks only in rows
+    padded like this; packed, they stay on the vector kernels (test_gpu_gguf.py)."""
     w = random_gguf_rows(t, rows, k, rng)
     pad = -w.shape[1] % 4
     return np.concatenate([w, np.zeros((rows, pad), np.uint8)], 1), w
@@ -287,6 +289,40 @@ def test_offset_activations(oracle, qtype, n):
     ops.ref_gemm_q(qtype, _dev(x), _dev(w), None, y, w.shape[1])
     # the types without an offset have 9.5e-8 here at most; 10 % for the two roundings more per block
     assert _err(y.cpu().numpy(), x.astype(np.float64) @ W.T) < 1.045e-7
+
+
+# The matrix cores' fp32 addition rounds down: without the blocks of negated
+# activations the mean error of these outputs is -5.9e-8 to -7.6e-8 of their rms
+# (measured), with them 4e-9 at most. 8192 or more outputs of an rms error of 9e-8
+# have a mean of 1e-9 by chance; a quarter of the smallest uncancelled one is the
+# bound. (Q3_K, Q6_K and IQ4_XS hardly show it, Q4_K and Q5_K have the offset's error
+# on top.) Rows off 16-byte alignment take the vector kernels: the sums of pieces are
+# to be no further from 64 bits than theirs.
+@pytest.mark.parametrize("fmt", [8, 18, "w4"])
+@pytest.mark.parametrize("n", [16, 40])
+def test_long_sums_have_no_bias(oracle, fmt, n):
+    rng = np.random.default_rng(n)
+    in_, out = 6144, 512
+    if fmt == "w4":
+        q = rng.integers(0, 256, (out, in_ // 2), dtype=np.uint8)
+        s = rng.uniform(0.001, 0.02, (out, in_ // 128)).astype(np.float32)
+        W = oracle.dequant_int4_rows(q, s, in_, 128).astype(np.float64)
+        run = lambda x, y: ops.ref_gemm_w4a16(x, _dev(q), _dev(s), None, y, 128)
+    else:
+        w = random_gguf_rows(fmt, out, in_, rng)
+        W = oracle.gguf_dequant_rows(fmt, w, out, in_).astype(np.float64)
+        run = lambda x, y: ops.ref_gemm_q(fmt, x, _dev(w), None, y, w.shape[1])
+    x = rng.standard_normal((n, in_)).astype(np.float32)
+    ref = x.astype(np.float64) @ W.T
+    err = []
+    for off in (0, 1):
+        xd = torch.zeros(n * in_ + 1, device="cuda")[off:off + n * in_].view(n, in_)
+        xd.copy_(torch.from_numpy(x))
+        y = torch.full((n, out), float("nan"), device="cuda")
+        run(xd, y)
+        err.append((y.cpu().numpy() - ref) / np.sqrt((ref ** 2).mean()))
+    assert abs(err[0].mean()) < 1.5e-8
+    assert np.sqrt((err[0] ** 2).mean()) < np.sqrt((err[1] ** 2).mean())
 
 
 def test_unaligned_elementwise(oracle):
