@@ -13,13 +13,14 @@
 // int8 activations use the int8 MFMA (exact int32 sums per 32 K), then the
 // weight scale and the activation block's scale in fp32.
 // The matrix cores' fp32 addition rounds down rather than to nearest (mean
-// error of a 6144-long product -0.67e-7 of its rms, against 0.68e-7 of spread),
-// and a sum of many such pieces drifts: every second 32-K block is computed
-// with negated activations and the scale's sign flipped, which cancels it.
+// error of 6144-long products -6e-8 to -8e-8 of their rms with Q8_0, IQ3_XXS and
+// int4 weights, against 9e-8 of spread), and a sum of many such pieces drifts:
+// every second 32-K block is computed with negated activations and the scale's
+// sign flipped, which leaves 4e-9 at most.
 // The partial products of a chunk (256 K; 128 where a chunk is that) are
 // added first, then the chunk sums: a two-level sum, whose rounding error
-// stays that of the vector kernels' lane sums (measured against 64 bits:
-// tests/test_gpu_splitmm.py).
+// (8.6e-8 to 1.15e-7 of the rms over the types at K 6144) is no larger than the
+// vector kernels' (tests/test_gpu_splitmm.py holds bias and error to that).
 //
 // Operands: A = activations (D row = token), B = weights (D column = weight
 // row), so a lane's outputs belong to one weight row and need one scale.
@@ -567,7 +568,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
                 if constexpr (T == 8 && MODE != kSmDense) {
                     // Clears what the epilogue recomputes anyway, for the branch's sake: without
                     // it the compiler no longer mixes these kernels' decode with the products
-                    // (1024 x 512 x 8, top-2, 40 tokens: 47 -> 53 us).
+                    // (2048 x 512 x 64, top-4, 1000 tokens: 213 -> 227 us).
                     float chk = 0.0f;
 #pragma unroll
                     for (int u = 0; u < 8; ++u) chk += l[u];
@@ -607,9 +608,9 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
     // int8 products mostly feed the int8 quantizer again, where one rounding more
     // or less moves a code: up to 16 rows per expert (gate/up) and in the linears'
     // tiles of at most 32 tokens the exact integer dots are scaled and added in
-    // 64 bits (a fused multiply-add costs the same), so the result is the rounded
-    // exact value: the int8 layer's error against 64 bits 5e-5 -> 1.3e-7, 64
-    // tokens 855 -> 873 us.
+    // 64 bits (64 tokens 855 -> 873 us), so the result is the rounded exact value
+    // and fewer codes move. A block of 64 tokens is 1.5e-7 from 64 bits where none
+    // does and about 5e-5 where one does, on some inputs with sums in 32 bits.
     constexpr bool F64 = I8 && ((SM && MODE == kSmGateUp) || (TB == 1 && MODE == kSmDense));
     using Acc = std::conditional_t<F64, double, float>;
     Acc acc[NK][TB][NV];

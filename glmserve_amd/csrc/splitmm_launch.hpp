@@ -17,13 +17,20 @@ static int sm_go(const SmArgs& a, unsigned gx, hipStream_t s) {
 }
 
 // K staged at a time for tiles of nt tokens; less where a row's chunk is wide, so
-// that two workgroups' LDS fits a CU (all but the 8- and 16-token expert tiles of
-// Q6_K with fp32 rows: 84 and 85 KiB).
+// that two 4-wave workgroups' LDS fits a CU (all but the 8- and 16-token expert tiles
+// of Q6_K with fp32 rows: 84 and 85 KiB). The linears' 8-wave workgroups of 16 and 32
+// fp32 rows (86 to 155 KiB) have a CU to themselves, and those of Q6_K with 4 fp32 or
+// 32 int8 rows (83 KiB).
 constexpr int sm_kx(uint32_t t, int nt) {
     const int k = nt <= 8 ? 128 : 64;
     return t == 12 || t == 13 || t == 14 ? k / 2 : k;
 }
 
+// The tiles of 4 to 16 and the 32-token ones of the IQ types, Q8_0 and Q3_K keep
+// everything in registers. Spilled to scratch, in registers: 32-token tiles of Q4_K
+// (fp32 14), Q5_K (fp32 43, int8 15) and Q6_K (fp32 17, int8 40), 64-token tiles up
+// to 3 with int8 rows, 7 to 17 with fp32; faster than the smaller tiles all the same
+// where gg_sm_tile takes them.
 // -2: a tile that no call of this type takes (sm_large_tile).
 template <uint32_t T, int MODE, bool I8>
 static int sm_moe_mode(int tile, const SmArgs& a, unsigned tiles, hipStream_t s) {
