@@ -100,7 +100,9 @@ constexpr bool sm_min(uint32_t t) { return t == 12 || t == 13; }          // wei
 // checkpoint's weights centre on zero, so what is left of the offset is small and
 // activations with a mean do not make two large sums cancel (fp32 rows of mean and
 // spread 1, K 6144, error against 64 bits: 1.1e-7 -> 9.4e-8, vector kernels 8.3e-8;
-// of mean 0: 1.2e-7 -> 1.0e-7, vector kernels 1.4e-7).
+// of mean 0: 1.2e-7 -> 1.0e-7, vector kernels 1.4e-7). Sums in 64 bits do not need
+// it (MID false; int8 linears of K 6144, 1 / 64 tokens: Q4_K 11.5 / 23.0 -> 11.1 / 22.7 us,
+// Q5_K 12.8 / 24.5 -> 12.2 / 23.8).
 constexpr uint32_t sm_mid(uint32_t t) { return t == 12 ? 8 : t == 13 ? 16 : 0; }
 constexpr int sm_kc(uint32_t t) { return t == 8 || t == kSmFp8 ? 128 : 256; }   // K per chunk
 constexpr int sm_cb(uint32_t t) {                                          // bytes per chunk of a row
@@ -216,8 +218,8 @@ __device__ __forceinline__ void sm_scale(const uint8_t* b, int ib, int j, float&
 }
 
 // Codes K = 32 ib + 8 f + [0, 8) of a chunk as 8 int8 (the types whose codes
-// are plain bit fields), the integers of gg_dec8i (less sm_mid). skew: b & 2.
-template <uint32_t T>
+// are plain bit fields), the integers of gg_dec8i (MID: less sm_mid). skew: b & 2.
+template <uint32_t T, bool MID>
 __device__ __forceinline__ void sm_codes(const uint8_t* b, int ib, int f, uint32_t skew, uint32_t& w0,
                                          uint32_t& w1) {
     if constexpr (T == 8) {   // 34-byte blocks in a 4-byte aligned chunk
@@ -232,10 +234,11 @@ __device__ __forceinline__ void sm_codes(const uint8_t* b, int ib, int f, uint32
             w0 |= ((sm_ld32(b + 16 + 8 * f) >> ib) & 0x01010101u) << 4;
             w1 |= ((sm_ld32(b + 20 + 8 * f) >> ib) & 0x01010101u) << 4;
         }
-        // less sm_mid per byte: 0..31 with bit 7 set borrows nothing from its neighbour
-        constexpr uint32_t mid = sm_mid(T) * 0x01010101u;
-        w0 = ((w0 | 0x80808080u) - mid) ^ 0x80808080u;
-        w1 = ((w1 | 0x80808080u) - mid) ^ 0x80808080u;
+        if constexpr (MID) {   // per byte: 0..31 with bit 7 set borrows nothing from its neighbour
+            constexpr uint32_t mid = sm_mid(T) * 0x01010101u;
+            w0 = ((w0 | 0x80808080u) - mid) ^ 0x80808080u;
+            w1 = ((w1 | 0x80808080u) - mid) ^ 0x80808080u;
+        }
     } else if constexpr (T == 14) {
         const int half = ib >> 2, qr = ib & 3;
         const uint8_t* ql = b + 64 * half + 32 * (qr & 1) + 8 * f;
@@ -299,7 +302,7 @@ __device__ __forceinline__ u32x4 sm_codes_bf16(const uint8_t* b, int ib, int f, 
         }
     } else {
         uint32_t w0, w1, a0, a1, a2, a3;
-        sm_codes<T>(b, ib, f, skew, w0, w1);
+        sm_codes<T, true>(b, ib, f, skew, w0, w1);
         sm_i8_bf16(w0, a0, a1);
         sm_i8_bf16(w1, a2, a3);
         w = u32x4{a0, a1, a2, a3};
@@ -318,7 +321,7 @@ __device__ __forceinline__ uint32_t sm_iq4nl4(uint32_t q) {
 }
 
 // The same codes as 8 int8.
-template <uint32_t T>
+template <uint32_t T, bool MID>
 __device__ __forceinline__ sm_i32x2 sm_codes_i8(const uint8_t* b, int ib, int f, uint32_t skew,
                                                 const SmTables<T, true>& L) {
     if constexpr (T == 18) {
@@ -333,7 +336,7 @@ __device__ __forceinline__ sm_i32x2 sm_codes_i8(const uint8_t* b, int ib, int f,
         return sm_i32x2{(int)sm_iq4nl4(sm_ld32(q) >> sh), (int)sm_iq4nl4(sm_ld32(q + 4) >> sh)};
     } else {
         uint32_t w0, w1;
-        sm_codes<T>(b, ib, f, skew, w0, w1);
+        sm_codes<T, MID>(b, ib, f, skew, w0, w1);
         return sm_i32x2{(int)w0, (int)w1};
     }
 }
@@ -649,7 +652,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
             else sm_scale<T>(b, i, 0, ds, dm);
             if constexpr (T == kSmW4)   // group: a multiple of 32
                 ds = a.sc[(size_t)(ob[r / 32] + (r & 31)) * (K / a.group) + (cc * KC + 32 * i) / a.group];
-            if constexpr (sm_min(T)) dm = __builtin_fmaf(-(float)sm_mid(T), ds, dm);
+            if constexpr (sm_min(T) && !F64) dm = __builtin_fmaf(-(float)sm_mid(T), ds, dm);
             // negative for the blocks whose fp32 activations are staged negated
             L.ds[wave][r][i] = !I8 && ((sm_g16(T) ? i / 2 : i) & 1) ? -ds : ds;
             if constexpr (sm_min(T)) L.dm[wave][r][i] = dm;
@@ -683,7 +686,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
 #pragma unroll
             for (int h = 0; h < HV; ++h) ds[h] = scale_of(nb, HV * ib + h);
             if constexpr (I8) {
-                const sm_i32x2 w = sm_codes_i8<T>(rb_, ib, lq, skew, L.tab);
+                const sm_i32x2 w = sm_codes_i8<T, !F64>(rb_, ib, lq, skew, L.tab);
                 Acc v[NV];
 #pragma unroll
                 for (int h = 0; h < HV; ++h) {
@@ -742,7 +745,7 @@ __global__ __launch_bounds__(64 * RW * KW, 2) void splitmm_kernel(SmArgs a) {
             for (int nb = 0; nb < NK; ++nb)
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
-                    w[nb][j] = sm_codes_i8<T>(brow + nb * BR * RS, ib, sm_g16(T) ? 2 * j + hh : 2 * hh + j, skew, L.tab);
+                    w[nb][j] = sm_codes_i8<T, !F64>(brow + nb * BR * RS, ib, sm_g16(T) ? 2 * j + hh : 2 * hh + j, skew, L.tab);
 #pragma unroll
             for (int tb = 0; tb < TB; ++tb) {
                 if (TB > 1 && tb >= ntb) continue;

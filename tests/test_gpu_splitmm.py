@@ -291,6 +291,32 @@ def test_offset_activations(oracle, qtype, n):
     assert _err(y.cpu().numpy(), x.astype(np.float64) @ W.T) < 1.045e-7
 
 
+# int8 linears of at most 32-token tiles and gate/up of at most 16 rows add the exact
+# integer dots in 64 bits: the result is the exact value rounded once, offsets included.
+# (Scales and offsets are exact in fp32; the reference adds both parts in 64 bits, where
+# dequantized fp32 weights would be rounded.) 1e-3: the 64-bit sums' own error beside a tie.
+@pytest.mark.parametrize("qtype", [8, 12, 13, 14])
+@pytest.mark.parametrize("n", [1, 16, 32])
+def test_int8_linears_round_once(oracle, qtype, n):
+    rng = np.random.default_rng(qtype + n)
+    in_, out = 2304, 512
+    w = random_gguf_rows(qtype, out, in_, rng)
+    if qtype in (12, 13):
+        parts = []
+        for zero in (slice(2, 4), slice(0, 2)):   # ds * q, then -dm
+            b = w.copy().reshape(out, in_ // 256, -1)
+            b[:, :, zero] = 0
+            parts.append(oracle.gguf_dequant_rows(qtype, b.reshape(w.shape), out, in_).astype(np.float64))
+        W = parts[0] + parts[1]
+    else:
+        W = oracle.gguf_dequant_rows(qtype, w, out, in_).astype(np.float64)
+    xq, xs, xd = _quant((rng.standard_normal((n, in_)) + 1).astype(np.float32))
+    y = torch.full((n, out), float("nan"), device="cuda")
+    wp = np.concatenate([w, np.zeros((out, -w.shape[1] % 4), np.uint8)], 1)
+    ops.ref_gemm_q_i8(qtype, xq, xs, _dev(wp), None, y, wp.shape[1])
+    assert (y.cpu().numpy() != (xd @ W.T).astype(np.float32)).mean() < 1e-3
+
+
 # The matrix cores' fp32 addition rounds down: without the blocks of negated
 # activations the mean error of these outputs is -5.9e-8 to -7.6e-8 of their rms
 # (measured), with them 4e-9 at most. 8192 or more outputs of an rms error of 9e-8
