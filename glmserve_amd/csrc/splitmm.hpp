@@ -101,8 +101,8 @@ constexpr bool sm_min(uint32_t t) { return t == 12 || t == 13; }          // wei
 // activations with a mean do not make two large sums cancel (fp32 rows of mean and
 // spread 1, K 6144, error against 64 bits: 1.1e-7 -> 9.4e-8, vector kernels 8.3e-8;
 // of mean 0: 1.2e-7 -> 1.0e-7, vector kernels 1.4e-7). Sums in 64 bits do not need
-// it (MID false; int8 linears of K 6144, 1 / 64 tokens: Q4_K 11.5 / 23.0 -> 11.1 / 22.7 us,
-// Q5_K 12.8 / 24.5 -> 12.2 / 23.8).
+// it (MID false; int8 linears, 6144 -> 2048, 1 / 64 tokens, us: Q4_K 11.8 / 23.3 centred,
+// 11.5 / 22.8 not; Q5_K 12.8 / 25.0 and 12.2 / 24.1).
 constexpr uint32_t sm_mid(uint32_t t) { return t == 12 ? 8 : t == 13 ? 16 : 0; }
 constexpr int sm_kc(uint32_t t) { return t == 8 || t == kSmFp8 ? 128 : 256; }   // K per chunk
 constexpr int sm_cb(uint32_t t) {                                          // bytes per chunk of a row
