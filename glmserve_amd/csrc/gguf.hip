@@ -918,9 +918,19 @@ static int gg_reduce(const GgMoeArgs& a, float* out, hipStream_t s) {
 // above the vector kernels'. int8 calls below
 // 2048 routed rows stay on the small tiles, whose sums do not depend on the
 // tile: grouped and ungrouped calls agree bit for bit there.
+// Narrow layers of few experts have few of the large workgroups (128 features x
+// tile), so fp32 rows take 16-row tiles where gate/up has less than 64 of them
+// (1024 x 512 x 8, top-2, n = 24 / 120, IQ4_XS: 25 / 30 us against 52 / 54, vector kernels
+// 46 / 108; the limit could be twice that on some layers and not on others: 6144 x 256 x
+// 64, top-8, n = 120: 231 against 176), and int8 rows 32 instead of 64 below one
+// per CU (2048 x 512 x 32, top-4, n = 600: 105 against 122, before these kernels 106;
+// with 856 of them, 2048 x 1024 x 64, top-8: 289 against 278).
 // Too little work: the vector kernels' 16-row workgroups win at n = 1 of that
 // layer with IQ types (71 against 77 us) and on small layers (2048 x 512,
-// top-4, n = 1: 17 against 26 us, n = 16: 72 against 41).
+// top-4, n = 1: 17 against 26 us, n = 16: 72 against 41). They are also
+// faster, but further from 64 bits (block error at n = 16 1.83e-7 against 1.64e-7), and
+// not taken, for fp32 IQ rows at width 256 ungrouped or about one to an expert
+// (6144 x 256 x 256, top-8, n = 16: 187 against 232, n = 20: 233 against 231).
 template <bool I8>
 static int gg_sm_tile(const GgMoeArgs& a, bool grouped) {
     const uint32_t gt = a.gate_type, dt = a.down_type;
@@ -930,19 +940,23 @@ static int gg_sm_tile(const GgMoeArgs& a, bool grouped) {
         !gg_aligned(a.up_q, a.up_rb, nullptr, 1) ||
         !gg_sm_ok(dt, a.down_q, a.down_rb, I8 ? (const void*)a.hq : (const void*)a.h_act, I8 ? 4 : 16, a.I, a.H))
         return 0;
-    const bool iq = gt == 18 || gt == 23;
+    auto kquant = [](uint32_t t) { return t >= 11 && t <= 14; };
+    const bool iq = gt == 18 || gt == 23, kq = kquant(gt) || kquant(dt);
     const long work = (long)nk * (a.I / 32) * (a.H / 256);
     if (nk <= E && work < (iq ? 24576 : 2048)) return 0;
     if (!grouped || nk <= E) return 4;
     if (nk <= 4 * E) return 8;
     if (I8 && nk < 2048) return 16;
-    auto kquant = [](uint32_t t) { return t >= 11 && t <= 14; };
     const bool large = sm_large_tile(gt, I8) && sm_large_tile(dt, I8);
-    if (kquant(gt) || kquant(dt)) {
+    if (kq) {
         const bool long16 = (sm_g16(gt) && a.H > 4096) || (sm_g16(dt) && a.I > 4096);
         return nk <= 16 * E || long16 ? 16 : kSmMidTile;
     }
-    return nk <= (I8 ? 16 : 64) * E || !large ? kSmMidTile : kSmLargeTile;
+    // gate/up workgroups for tiles of t rows, the last of each expert half full
+    auto wgs = [&](int t) { return (long)(nk / t + E / 2) * ((a.I + 127) / 128); };
+    if (!I8 && wgs(kSmMidTile) < 64) return 16;
+    if (!large || nk <= (I8 ? 16 : 64) * E || (I8 && wgs(kSmLargeTile) < 256)) return kSmMidTile;
+    return kSmLargeTile;
 }
 
 // Gate/up and down on splitmm_kernel; d: the grouping in tiles of `tile` rows.

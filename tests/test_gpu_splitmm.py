@@ -103,10 +103,12 @@ def test_gemm_w4_fp8(oracle, n, in_, out, g):
     assert _err(y.cpu().numpy(), x.astype(np.float64) @ W.T) < 2.5e-7
 
 
-# E = 8, top-4: ungrouped (tiles of 4 with one row), then 12, 36, 280 and 2080
-# routed rows grouped (tiles of 8, 16 or 32, 32 and 64), ids outside [0, E) among them.
+# E = 8, top-4: ungrouped (tiles of 4 with one row), then 12, 36, 280, 400, 2080 and 3840
+# routed rows grouped (tiles of 8, 16, 16, 32, 32 or 64 and 64; int8 16 up to 2047 rows,
+# then 32), ids outside [0, E) among them.
 @pytest.mark.parametrize("types", [(18, 18, 23), (8, 8, 8), (12, 12, 13), (11, 11, 14), (23, 23, 18)])
-@pytest.mark.parametrize("n,grouped", [(3, False), (3, True), (9, True), (70, True), (520, True)])
+@pytest.mark.parametrize("n,grouped", [(3, False), (3, True), (9, True), (70, True), (100, True),
+                                       (520, True), (960, True)])
 def test_moe(oracle, types, n, grouped):
     H, I, E, k = 1024, 512, 8, 4
     rng = np.random.default_rng(sum(types) + n)
@@ -237,10 +239,10 @@ def test_extreme_activations_large_tiles(oracle, qtype):
     assert _err(got[ok], x[ok].astype(np.float64) @ W.T) < TOL[qtype]
 
 
-# Tiles of 4 (ungrouped), 8 or 16, and 32 rows: gate and up of a token with an infinity,
+# Tiles of 4 (ungrouped), 16 and 32 rows: gate and up of a token with an infinity,
 # and of one whose sums of codes overflow.
 @pytest.mark.parametrize("types", [(18, 18, 23), (12, 12, 14), (14, 14, 8)])
-@pytest.mark.parametrize("n,grouped", [(3, False), (9, True), (70, True)])
+@pytest.mark.parametrize("n,grouped", [(3, False), (9, True), (100, True)])
 def test_moe_extreme_activations(oracle, types, n, grouped):
     H, I, E, k = 1024, 512, 8, 4
     rng = np.random.default_rng(sum(types) + n)
